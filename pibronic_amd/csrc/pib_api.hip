@@ -20,8 +20,9 @@ namespace pib {
 // Per-mode constant records of the lanes kernel (layout: ModeRec). Rebuilt by the coupling
 // and O-matrix set setters once the coupling and the rho and vib sets agree in shape; the
 // +-dbeta entries stay zero until those sets are given.
+int rebuild_block_table(pib_ctx* c);
 int rebuild_mode_table(pib_ctx* c) {
-  c->mode_tab_ok = false;
+  c->mode_tab_ok = c->block_ok[0] = c->block_ok[1] = false;
   const int A = c->A, N = c->N, AR = c->set_A[SET_RHO];
   if (!c->coupling_set || !AR || c->set_A[SET_VIB] != A || c->set_N[SET_RHO] != N || c->set_N[SET_VIB] != N)
     return PIB_OK;
@@ -67,7 +68,121 @@ int rebuild_mode_table(pib_ctx* c) {
   if ((r = upload(c, c->mode_tab, tab.data(), tab.size() * sizeof(double)))) return r;
   if ((r = upload(c, c->mode_tab_f, tabf.data(), tabf.size() * sizeof(float)))) return r;
   c->mode_tab_ok = true;
+  return rebuild_block_table(c);
+}
+
+// Constants of the block kernel, rebuilt by the setters once the coupling, the rho and vib sets
+// and the beads agree (in the usual order of calls once, when the beads are set).
+int rebuild_block_table(pib_ctx* c) {
+  c->block_ok[0] = c->block_ok[1] = false;
+  const int A = c->A, N = c->N, AR = c->set_A[SET_RHO];
+  if (!c->mode_tab_ok || c->P < 3 || A > kWideMaxStates || AR > kWideMaxStates) return PIB_OK;
+  if (A < 5 && eval_supported(A, AR)) return PIB_OK;  // never routed to the block kernel
+  BlockModel m{};
+  m.A = A;
+  m.AR = AR;
+  m.N = N;
+  m.tau = c->tau;
+  m.energy = c->h_energy.data();
+  m.linear = c->h_linear.data();
+  m.qdiag = c->h_qdiag.empty() ? nullptr : c->h_qdiag.data();
+  m.pairs = c->h_pairs;
+  m.qpair = c->h_qpair.data();
+  for (int pm = 0; pm < 2; ++pm) {
+    for (int s = 2 * pm; s < 2 * pm + 2; ++s) {
+      if (c->set_A[s] != (s == SET_RHO ? AR : A) || c->set_N[s] != N) return PIB_OK;
+      m.set[s] = {c->set_A[s],         c->h_th[s].data(), c->h_cs[s].data(),
+                  c->h_lin[s].data(), c->h_k2[s].data(), c->h_lpref[s].data()};
+    }
+    BlockTables& t = c->block[pm];
+    t = block_tables(m, pm != 0);
+    const int r = upload(c, c->block_tab[pm], t.data.data(), t.data.size() * sizeof(double));
+    std::vector<double>().swap(t.data);
+    if (r) return r;
+    c->block_ok[pm] = true;
+  }
   return PIB_OK;
+}
+
+// The block kernel takes every (A, A_rho) without a lanes kernel (without +-dbeta up to eight
+// surfaces), and of those with one the sizes where it is the faster: A = 8, and with +-dbeta
+// (three ring chains in one lane's registers) A = 7. Measured (MI355X, us, lanes / block, N = 2 A, P = 64): A = 8 1,000 samples 46 / 27, 16,384
+// 388 / 237, 1e5 1650 / 1416; with +-dbeta 1e5 5470 / 1882; A = 7 1e5 1219 / 1290, with +-dbeta
+// 16,384 837 / 286, 1e5 3163 / 1706; A = 6 1e5 732 / 1235, with +-dbeta 1458 / 1595.
+bool uses_block(const pib_ctx* c, int flags) {
+  const bool pm = (flags & PIB_EVAL_PM) != 0;
+  if (!c->block_ok[pm] || (flags & (PIB_EVAL_WIDE | PIB_EVAL_FP32 | PIB_EVAL_BF16X3))) return false;
+  for (int s = 0; s < (pm ? 4 : 2); ++s)
+    if (!c->pref_positive[s]) return false;  // it works with log F_a
+  if (!eval_supported(c->A, c->set_A[SET_RHO])) return pm || block_size(c->A, c->set_A[SET_RHO]) <= 8;
+  return c->A >= (pm ? 7 : 8);
+}
+
+// Bead streams per sample (1, 2 or 4) of the block kernel: more of them fill the chip with fewer
+// samples, at the price of joining the streams' chains and, where P / C is no multiple of four, of
+// partly empty steps of the front. The estimate is a wave's steps (front and back about 2 : 3) plus
+// the joins, times the waves per SIMD; below four of them latency shows: one wave takes about 1.6
+// times its share, two 2.4, three 3.2. Measured (MI355X, us at C = 1 / 2 / 4): A=8 N=16 P=64 1,000
+// samples 85 / 46 / 27, 4,000 121 / 81 / 71, 8,000 160 / 137 / 134, 16,384 242 / 240 / 237, 1e5
+// 1416 / 1420 / 1416; A=11 N=17 P=50 with +-dbeta 3,001 samples 164 / 149 / 128, 16,384
+// 579 / 591 / 649; A=16 N=10 P=30 with +-dbeta 20,000 samples 1151 / 1089 / 1158.
+static int block_streams(int num_cu, int64_t B, int P) {
+  const double simds = 4.0 * num_cu;
+  int best = 1;
+  double least = 0.0;
+  for (int C = 1; C <= 4; C *= 2) {
+    const int K = (P + C - 1) / C;
+    const double per_simd = std::ceil((double)((B * C + 3) / 4) / simds);
+    const double cost = (0.4 * (4 * ((K + 3) / 4)) + 0.6 * K + (C - 1) * 0.8) *
+                        (per_simd < 4.0 ? 0.8 * per_simd + 0.8 : per_simd);
+    if (C == 1 || cost < least) {
+      best = C;
+      least = cost;
+    }
+  }
+  return best;
+}
+
+static BlockArgs block_args(const pib_ctx* c, const EvalArgs& a, bool pm) {
+  BlockArgs b{};
+  b.q = a.q;
+  b.qf = a.qf;
+  b.qcentre = a.qcentre;
+  b.B = a.B;
+  b.N = a.N;
+  b.P = a.P;
+  b.A = a.A;
+  b.AR = a.AR;
+  const BlockTables& k = c->block[pm];
+  b.S = k.S;
+  b.C = block_streams(c->num_cu, a.B, a.P);
+  b.K = (a.P + b.C - 1) / b.C;
+  b.noscale = a.noscale;
+  b.quad = a.qdiag != nullptr;
+  b.npair = a.npair;
+  b.ldiag = k.ldiag;
+  b.op_pairs = k.op_pairs;
+  b.pair = a.pair;
+  const double* t = (const double*)c->block_tab[pm].p;
+  b.energy = t + k.energy;
+  b.k2 = t + k.k2;
+  b.lpref = t + k.lpref;
+  b.tcs = t + k.tcs;
+  b.ops = t + k.ops;
+  b.cpair = t + k.cpair;
+  b.out = a.out;
+  b.out_stride = a.out_stride;
+  b.dbg = a.dbg;
+  return b;
+}
+
+hipError_t launch_eval(const pib_ctx* c, int flags, bool wide, const EvalArgs& a, hipStream_t s) {
+  const int pm = (flags & PIB_EVAL_PM) ? 1 : 0;
+  if (flags & PIB_EVAL_FP32) return launch_eval_fp32(a.A, a.AR, pm, a, s);
+  if (uses_block(c, flags)) return launch_eval_block(pm, block_args(c, a, pm != 0), s);
+  if (wide) return launch_eval_wide(pm, a, s, (flags & PIB_EVAL_BF16X3) != 0);
+  if (a.qf) return launch_eval_fp64_offsets(a.A, a, s);
+  return launch_eval_fp64(a.A, a.AR, pm, a, s);
 }
 
 int make_eval_args(pib_ctx* c, int flags, int64_t B, EvalArgs* out_args, bool* wide_out) {
@@ -212,6 +327,8 @@ int pib_ctx_destroy(pib_ctx* c) {
     release(c->k2_f[s]);
   }
   release(c->mode_tab);
+  release(c->block_tab[0]);
+  release(c->block_tab[1]);
   release(c->fb_mu);
   release(c->fb_c);
   release(c->fb_qidx);
@@ -273,7 +390,10 @@ int pib_set_coupling(pib_ctx* c, int A, int N, const double* E, const double* L,
   }
   c->has_qdiag = any_diag;
   if (any_diag && (r = upload(c, c->qdiag, qd.data(), qd.size() * sizeof(double)))) return r;
+  c->h_energy.assign(E, E + AA);
   c->h_linear.assign(L, L + (size_t)N * AA);
+  c->h_pairs = pairs;
+  c->h_qpair = qp;
   if (any_diag) c->h_qdiag = qd; else c->h_qdiag.clear();
   c->npair = (int)(pairs.size() / 2);
   if (c->npair) {
@@ -351,6 +471,8 @@ int pib_set_omatrix_set(pib_ctx* c, int slot, int A_set, int N, const double* co
     if ((r = upload(c, c->lpref[slot], lp.data(), A_set * sizeof(double)))) return r;
     std::vector<float> k2f(k2.begin(), k2.end());
     if ((r = upload(c, c->k2_f[slot], k2f.data(), A_set * sizeof(float)))) return r;
+    c->h_k2[slot] = k2;
+    c->h_lpref[slot] = lp;
     c->h_th[slot] = th;
     c->h_cs[slot].assign(csch, csch + N);
     c->h_lin[slot] = lin;
@@ -383,7 +505,7 @@ int pib_set_beads(pib_ctx* c, int P, double tau) {
   if (!std::isfinite(tau) || tau <= 0.0) return fail(c, PIB_ERR_ARG, "set_beads: tau must be > 0");
   c->P = P;
   c->tau = tau;
-  return PIB_OK;
+  return rebuild_block_table(c);
 }
 
 int pib_set_lanes_per_sample(pib_ctx* c, int lanes) {
@@ -416,10 +538,7 @@ int pib_eval_block(pib_ctx* c, const double* q, int64_t B, int flags, double* ou
   a.out_stride = out_stride;
   a.dbg = dbg;
   PIB_HIP(c, hipSetDevice(c->device));
-  const int pm = (flags & PIB_EVAL_PM) ? 1 : 0;
-  hipError_t e = (flags & PIB_EVAL_FP32) ? launch_eval_fp32(c->A, a.AR, pm, a, (hipStream_t)stream)
-                 : wide ? launch_eval_wide(pm, a, (hipStream_t)stream, (flags & PIB_EVAL_BF16X3) != 0)
-                                         : launch_eval_fp64(c->A, a.AR, pm, a, (hipStream_t)stream);
+  const hipError_t e = launch_eval(c, flags, wide, a, (hipStream_t)stream);
   if (e != hipSuccess) return hip_fail(c, e, "eval_block launch");
   return PIB_OK;
 }
@@ -446,7 +565,7 @@ int pib_eval_block_flow_offsets(pib_ctx* c, const float* dq, int64_t B, int flag
   a.out = out;
   a.out_stride = out_stride;
   PIB_HIP(c, hipSetDevice(c->device));
-  hipError_t e = launch_eval_fp64_offsets(c->A, a, (hipStream_t)stream);
+  const hipError_t e = launch_eval(c, flags, false, a, (hipStream_t)stream);
   if (e != hipSuccess) return hip_fail(c, e, "eval_block_flow_offsets launch");
   return PIB_OK;
 }

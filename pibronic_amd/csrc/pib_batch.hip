@@ -50,6 +50,7 @@ struct pib_batch {
   LaneProbs lprobs{};          // the lanes family's kernel-argument copy of args
   bool lane_ok = false, wide_ok = false;
   bool seq_lanes = true;  // every problem has a compiled lanes kernel (one launch per problem)
+  std::vector<bool> wide;  // problems without one
   int A = 0, AR = 0;
   // schedule
   int family = 0;  // PIB_BATCH_LANES or PIB_BATCH_WIDE
@@ -149,9 +150,7 @@ hipError_t launch_batch_eval(pib_batch* b, hipStream_t s) {
   if (b->family == PIB_BATCH_SEQUENTIAL) {  // one launch per problem, tuned lanes
     for (int i = 0; i < b->n; ++i) {
       const EvalArgs& a = b->args[i];
-      hipError_t e = (b->flags & PIB_EVAL_FP32) ? launch_eval_fp32(a.A, a.AR, b->pm, a, s)
-                     : b->seq_lanes             ? launch_eval_fp64(a.A, a.AR, b->pm, a, s)
-                                                : launch_eval_wide(b->pm, a, s);
+      const hipError_t e = launch_eval(b->ctx[i], b->flags, b->wide[i], a, s);
       if (e != hipSuccess) return e;
     }
     return hipSuccess;
@@ -277,6 +276,8 @@ int pib_batch_create(int n, pib_ctx* const* ctxs, int64_t B, int flags, double d
   b->args.resize(n);
   b->lanes.resize(n);
   b->gens.resize(n);
+  b->wide.resize(n);
+  bool all_block = true;
   for (int i = 0; i < n; ++i) {
     pib_ctx* c = ctxs[i];
     if (!c) return bfail(b, PIB_ERR_ARG, "batch_create: null context");
@@ -286,7 +287,9 @@ int pib_batch_create(int n, pib_ctx* const* ctxs, int64_t B, int flags, double d
       return bfail(b, PIB_ERR_STATE, "batch_create: problem " + std::to_string(i) + ": " + c->err);
     b->gens[i] = c->gen;
     const int A = c->A, AR = b->args[i].AR;
+    b->wide[i] = wide;
     if (wide) b->seq_lanes = false;
+    all_block = all_block && uses_block(c, flags);
     if (wide || (i > 0 && (A != b->A || AR != b->AR))) b->lane_ok = false;
     if (i == 0) { b->A = A; b->AR = AR; }
     if (A > kWideMaxStates || AR > kWideMaxStates) b->wide_ok = false;
@@ -310,7 +313,10 @@ int pib_batch_create(int n, pib_ctx* const* ctxs, int64_t B, int flags, double d
     b->args[i].out_stride = B;
     b->args[i].dbg = nullptr;
   }
+  // problems of the block kernel (pib_eval_block.hip) fill the chip one launch each; the
+  // persistent kernels of either family are slower for them
   b->family = (flags & PIB_EVAL_FP32) ? PIB_BATCH_SEQUENTIAL
+              : all_block             ? PIB_BATCH_SEQUENTIAL
               : b->lane_ok            ? PIB_BATCH_LANES
               : b->wide_ok            ? PIB_BATCH_WIDE
                                       : PIB_BATCH_SEQUENTIAL;
@@ -411,9 +417,7 @@ int pib_batch_eval_sequential(pib_batch* b, void* stream) {
     s.out = a.out;
     s.out_stride = a.out_stride;
     s.dbg = nullptr;
-    hipError_t e = (b->flags & PIB_EVAL_FP32) ? launch_eval_fp32(s.A, s.AR, b->pm, s, (hipStream_t)stream)
-                   : wide ? launch_eval_wide(b->pm, s, (hipStream_t)stream)
-                          : launch_eval_fp64(s.A, s.AR, b->pm, s, (hipStream_t)stream);
+    const hipError_t e = launch_eval(b->ctx[i], b->flags, wide, s, (hipStream_t)stream);
     if (e != hipSuccess) return bfail(b, PIB_ERR_HIP, std::string("batch_eval_sequential: ") + hipGetErrorString(e));
   }
   return PIB_OK;

@@ -71,6 +71,8 @@ struct CoordBuf {
   // and the value, formed where it is used
   __device__ __forceinline__ raw_t load(int j, int P, int p) const { return (*this)[j * P + p]; }
   __device__ __forceinline__ double value(int, raw_t r) const { return r; }
+  // the same in one step, for a mode that differs between lanes
+  __device__ __forceinline__ double value_at(int j, int P, int p) const { return load(j, P, p); }
   // the wave's samples [first, first + per_wave) (first made wave-uniform explicitly); `sample`
   // is this lane's sample, or -1 for a lane past the block (which reads the wave's first)
   __device__ __forceinline__ static CoordBuf wave_samples(const double* q, int64_t B, int64_t NP, int64_t first,
@@ -97,6 +99,7 @@ struct CoordOffsetBuf {
     return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, (base + j * P + p) * 4, 0, 0));
   }
   __device__ __forceinline__ double value(int j, raw_t r) const { return centre[j] + (double)r; }
+  __device__ __forceinline__ double value_at(int j, int P, int p) const { return centre[j] + (double)load(j, P, p); }
   __device__ __forceinline__ static CoordOffsetBuf wave_samples(const float* q, const double* c, int64_t B,
                                                                 int64_t NP, int64_t first, int per_wave,
                                                                 int64_t sample) {

@@ -42,6 +42,12 @@ struct pib_ctx {
   std::vector<double> h_linear, h_qdiag;
   pib::DevBuf mode_tab, mode_tab_f, k2_f[pib::NUM_SETS];
   bool mode_tab_ok = false;
+  // block kernel: its constants (block_tables) and the host copies they are built from
+  std::vector<double> h_energy, h_qpair, h_k2[pib::NUM_SETS], h_lpref[pib::NUM_SETS];
+  std::vector<int> h_pairs;
+  pib::DevBuf block_tab[2];     // without and with +-dbeta
+  pib::BlockTables block[2];    // section offsets; their data is dropped after the upload
+  bool block_ok[2] = {false, false};
   pib::DevBuf tc_f[pib::NUM_SETS], cs_f[pib::NUM_SETS], lpref_f[pib::NUM_SETS];
   bool pref_positive[pib::NUM_SETS] = {false, false, false, false};
   // beads
@@ -159,4 +165,9 @@ namespace pib {
 // every EvalArgs field except q, out, out_stride and dbg. Returns PIB_OK or an error code (with
 // the message in c->err); *wide tells which kernel family applies.
 int make_eval_args(pib_ctx* c, int flags, int64_t B, EvalArgs* a, bool* wide);
+// Launch the evaluation that make_eval_args prepared (flags as given there) with the kernel
+// this context's sizes call for; `a` complete with q (or qf), out, out_stride and dbg.
+hipError_t launch_eval(const pib_ctx* c, int flags, bool wide, const EvalArgs& a, hipStream_t s);
+// Whether launch_eval takes the block kernel for these flags.
+bool uses_block(const pib_ctx* c, int flags);
 }  // namespace pib

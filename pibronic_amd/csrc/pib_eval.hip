@@ -458,15 +458,8 @@ struct EvalOccupancy {
 
 // The samples of one wave: wave w evaluates samples [w * 64/G, (w + 1) * 64/G) of `args`.
 // QF: coordinates as float offsets from a per-mode centre (args.qf, args.qcentre).
-// CH (with PM): 0 accumulates the three ring chains of g, g+ and g- together; 1, 2, 3 only the
-// chain of g (writing rho, g and log S), of g+ or of g- (writing that output alone). Every pass
-// forms the same M and scaling as the three-chain form, so three passes give its outputs bit
-// for bit, with a third of the accumulators live (at A = 8 the three chains do not fit in the
-// registers of one lane).
-template <int A, int AR, bool PM, bool DBG, bool QF = false, int CH = 0>
+template <int A, int AR, bool PM, bool DBG, bool QF = false>
 __device__ __forceinline__ void eval_wave(const EvalArgs& args, int64_t wave) {
-  static_assert(CH == 0 || (PM && !DBG && !QF), "single-chain passes are +-dbeta passes without debug records");
-  constexpr bool ALL = PM && CH == 0;  // the g+ and g- chains beside g's
   const int lane = threadIdx.x & (kWave - 1);
   const int G = args.G, K = args.K, N = args.N, P = args.P;
   const int gl = lane & (G - 1);
@@ -501,7 +494,7 @@ __device__ __forceinline__ void eval_wave(const EvalArgs& args, int64_t wave) {
 #pragma unroll
     for (int k = 0; k < A; ++k) {
       Ng[i][k] = (i == k) ? 1.0 : 0.0;
-      if (ALL) { Np[i][k] = Ng[i][k]; Nm[i][k] = Ng[i][k]; }
+      if (PM) { Np[i][k] = Ng[i][k]; Nm[i][k] = Ng[i][k]; }
     }
   // log-domain products: lr[a] = sum_p log(O_rho,a(p) / S_p), ls = sum_p log S_p
   double lr[AR];
@@ -556,8 +549,8 @@ __device__ __forceinline__ void eval_wave(const EvalArgs& args, int64_t wave) {
     for (int a = 0; a < A; ++a) {
       lOv[a] = fma(-0.5, (tv + ev[a]) + sv.k2[a], sv.lpref[a]);
       lS = fmax(lS, lOv[a]);
-      if (ALL || CH == 2) lOp[a] = fma(-0.5, (tp + ep[a]) + sp.k2[a], sp.lpref[a]);
-      if (ALL || CH == 3) lOm[a] = fma(-0.5, (tm + em[a]) + sm.k2[a], sm.lpref[a]);
+      if (PM) lOp[a] = fma(-0.5, (tp + ep[a]) + sp.k2[a], sp.lpref[a]);
+      if (PM) lOm[a] = fma(-0.5, (tm + em[a]) + sm.k2[a], sm.lpref[a]);
     }
     if (args.noscale) lS = 0.0;
 
@@ -595,9 +588,8 @@ __device__ __forceinline__ void eval_wave(const EvalArgs& args, int64_t wave) {
     for (int a = 0; a < AR; ++a) lr[a] += lOr[a] - lS;
 #pragma unroll
     for (int a = 0; a < A; ++a) {
-      // in a single-chain pass Ov holds the factors of that pass's chain
-      Ov[a] = exp((CH == 2 ? lOp[a] : (CH == 3 ? lOm[a] : lOv[a])) - lS);
-      if (ALL) {
+      Ov[a] = exp(lOv[a] - lS);
+      if (PM) {
         Op[a] = exp(lOp[a] - lS);
         Om[a] = exp(lOm[a] - lS);
       }
@@ -609,7 +601,7 @@ __device__ __forceinline__ void eval_wave(const EvalArgs& args, int64_t wave) {
 #pragma unroll
       for (int c = 0; c < A; ++c) {
         rg[c] = Ng[i][c];
-        if (ALL) { rpl[c] = Np[i][c]; rmi[c] = Nm[i][c]; }
+        if (PM) { rpl[c] = Np[i][c]; rmi[c] = Nm[i][c]; }
       }
 #pragma unroll
       for (int k = 0; k < A; ++k) {
@@ -617,7 +609,7 @@ __device__ __forceinline__ void eval_wave(const EvalArgs& args, int64_t wave) {
 #pragma unroll
         for (int c = 1; c < A; ++c) s = fma(rg[c], M[c][k], s);
         Ng[i][k] = s * Ov[k];
-        if (ALL) {
+        if (PM) {
           double sp_ = rpl[0] * M[0][k], sm_ = rmi[0] * M[0][k];
 #pragma unroll
           for (int c = 1; c < A; ++c) {
@@ -655,7 +647,7 @@ __device__ __forceinline__ void eval_wave(const EvalArgs& args, int64_t wave) {
         }
       }
     }
-    if (ALL) {
+    if (PM) {
 #pragma unroll
       for (int w = 0; w < 2; ++w) {
         double (&X)[A][A] = (w == 0) ? Np : Nm;
@@ -689,13 +681,7 @@ __device__ __forceinline__ void eval_wave(const EvalArgs& args, int64_t wave) {
     if (leader) ls += tl;
   }
 
-  if (live && gl == 0 && CH >= 2) {  // the g+ or g- pass: the trace of its chain alone
-    double t = Ng[0][0];
-#pragma unroll
-    for (int i = 1; i < A; ++i) t += Ng[i][i];
-    args.out[(CH == 2 ? OUT_GP : OUT_GM) * args.out_stride + sample] = t;
-  }
-  if (live && gl == 0 && CH < 2) {
+  if (live && gl == 0) {
     const int64_t st = args.out_stride;
     double rho = exp(lr[0]);
 #pragma unroll
@@ -705,7 +691,7 @@ __device__ __forceinline__ void eval_wave(const EvalArgs& args, int64_t wave) {
     for (int i = 1; i < A; ++i) g += Ng[i][i];
     args.out[OUT_RHO * st + sample] = rho;
     args.out[OUT_G * st + sample] = g;
-    if (ALL) {
+    if (PM) {
       double gp = Np[0][0], gm = Nm[0][0];
 #pragma unroll
       for (int i = 1; i < A; ++i) { gp += Np[i][i]; gm += Nm[i][i]; }
@@ -720,13 +706,6 @@ template <int A, int AR, bool PM, bool DBG>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EvalOccupancy<A, PM>::waves)))
 k_eval_fp64(const EvalArgs args) {
   eval_wave<A, AR, PM, DBG>(args, ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kWave);
-}
-
-// one ring chain of the +-dbeta evaluation (CH 1: g with rho and log S, 2: g+, 3: g-)
-template <int A, int AR, int CH>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EvalOccupancy<A, true>::waves)))
-k_eval_fp64_chain(const EvalArgs args) {
-  eval_wave<A, AR, true, false, false, CH>(args, ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kWave);
 }
 
 // the same on float offsets from a per-mode centre (pib_eval_block_flow_offsets)
@@ -821,25 +800,18 @@ static hipError_t launch_a(int pm, const EvalArgs& a, hipStream_t s) {
   // while this kernel is bound by dependent FP64 arithmetic, not by memory.
   const EvalArgs& b = a;
   const size_t lds = 0;
-  if constexpr (A == 8 && AR == 8) {
-    // +-dbeta at A = 8: the three ring chains in three passes of one chain each (the three
-    // together spill 1.5 KB per lane to scratch: 5.78 ms against 3.55 ms for the passes at
-    // 65,536 samples, N = 16, P = 64, timed alone; in a block loop after evaluations without
-    // +-dbeta both forms have been measured at ~1.6x their cycles, the passes never slower; at
-    // A = 7 one pass is still faster, 2.00 ms against about three times the plain kernel's
-    // 0.77); the debug records keep the one-pass form
-    if (pm && !dbg) {
-      hipLaunchKernelGGL((k_eval_fp64_chain<A, AR, 1>), grid, dim3(threads), lds, s, b);
-      hipLaunchKernelGGL((k_eval_fp64_chain<A, AR, 2>), grid, dim3(threads), lds, s, b);
-      hipLaunchKernelGGL((k_eval_fp64_chain<A, AR, 3>), grid, dim3(threads), lds, s, b);
-      return hipGetLastError();
+  if (pm) {
+    // from A = 7 on +-dbeta runs in the block kernel (three ring chains beside the exponential do
+    // not fit in one lane's registers)
+    if constexpr (A < 7) {
+      if (dbg)
+        hipLaunchKernelGGL((k_eval_fp64<A, AR, true, true>), grid, dim3(threads), lds, s, b);
+      else
+        hipLaunchKernelGGL((k_eval_fp64<A, AR, true, false>), grid, dim3(threads), lds, s, b);
+    } else {
+      return hipErrorInvalidValue;
     }
-  }
-  if (pm && dbg)
-    hipLaunchKernelGGL((k_eval_fp64<A, AR, true, true>), grid, dim3(threads), lds, s, b);
-  else if (pm)
-    hipLaunchKernelGGL((k_eval_fp64<A, AR, true, false>), grid, dim3(threads), lds, s, b);
-  else if (dbg)
+  } else if (dbg)
     hipLaunchKernelGGL((k_eval_fp64<A, AR, false, true>), grid, dim3(threads), lds, s, b);
   else
     hipLaunchKernelGGL((k_eval_fp64<A, AR, false, false>), grid, dim3(threads), lds, s, b);
@@ -869,7 +841,10 @@ bool eval_supported(int A, int AR) {
 }
 
 hipError_t launch_eval_fp64(int A, int AR, int pm, const EvalArgs& a, hipStream_t s) {
-#define PIB_CASE(a_, ar_) if (A == a_ && AR == ar_) return launch_a<a_, ar_>(pm, a, s);
+  // A = 8 runs in the block kernel; here only its persistent batched form is compiled
+#define PIB_CASE(a_, ar_) \
+  if constexpr (a_ < 8)   \
+    if (A == a_ && AR == ar_) return launch_a<a_, ar_>(pm, a, s);
   PIB_EVAL_CASES(PIB_CASE)
 #undef PIB_CASE
   return hipErrorInvalidValue;
@@ -894,7 +869,6 @@ hipError_t launch_eval_fp64_offsets(int A, const EvalArgs& a, hipStream_t s) {
     case 5: return launch_offsets_a<5>(a, s);
     case 6: return launch_offsets_a<6>(a, s);
     case 7: return launch_offsets_a<7>(a, s);
-    case 8: return launch_offsets_a<8>(a, s);
   }
   return hipErrorInvalidValue;
 }

@@ -3,6 +3,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <vector>
+
 namespace pib {
 
 // One TemperatureDependentClass (pibronic/pimc/pimc.py:59-89) plus the state shift of the
@@ -172,6 +174,60 @@ struct BatchTile {
 hipError_t launch_eval_fp64(int A, int AR, int pm, const EvalArgs& a, hipStream_t s);
 hipError_t launch_eval_fp64_offsets(int A, const EvalArgs& a, hipStream_t s);
 hipError_t launch_eval_wide(int pm, const EvalArgs& a, hipStream_t s, bool bf16x3 = false);
+
+// Arguments of the block kernel (pib_eval_block.hip). The constants are in the operand order of
+// its matrix instructions: coupling elements (r, c), r >= c, numbered off-diagonal first, in
+// tiles of 16, and surfaces by register s * NB + I (surfaces 4I..4I+3 of O-matrix set s).
+struct BlockArgs {
+  const double* q;      // as EvalArgs
+  const float* qf;
+  const double* qcentre;
+  int64_t B;
+  int N, P, A, AR;
+  int S;                // the kernel's size, block_size(A, AR)
+  int C, K;             // bead streams per sample (1, 2, 4), beads per stream = ceil(P / C)
+  int noscale, quad, npair;
+  int ldiag;            // the linear couplings have elements beyond the off-diagonal tiles
+  int op_pairs;         // operand pairs per mode group
+  const int* pair;
+  const double* energy;  // [tile][e % 4][e / 4], e the element's row in its tile; times -tau
+  const double* k2;      // [register / 4][surface % 4][register % 4]
+  const double* lpref;   // the same; -inf for padded surfaces
+  const double* tcs;     // [mode][4 sets]{th, csch}
+  const double* ops;     // [mode / 4][operand / 2][16 (mode % 4) + row][operand % 2]; operands: the
+                         // O-exponents' linear parts (row 4 (register % 4) + surface % 4), linear and
+                         // quadratic couplings (row e), the rest of the linear ones; times -tau
+  const double* cpair;   // [pair / 4][tile][16 (pair % 4) + e], times -tau
+  double* out;
+  int64_t out_stride;
+  double* dbg;
+};
+// surfaces the block kernel is sized for (at least 5: smaller models have their own kernel)
+inline int block_size(int A, int AR) {
+  const int m = A > AR ? A : AR;
+  return m < 5 ? 5 : m;
+}
+hipError_t launch_eval_block(int pm, const BlockArgs& a, hipStream_t s);
+// Host model the block kernel's constants are built from.
+struct BlockModel {
+  int A, AR, N;
+  double tau;
+  const double* energy;  // A*A
+  const double* linear;  // N*A*A
+  const double* qdiag;   // N*A*A = 0.5*Q[j,j] or nullptr
+  std::vector<int> pairs;
+  const double* qpair;   // pairs/2 * A*A
+  struct Set {
+    int A;
+    const double *th, *cs, *lin, *k2, *lpref;
+  } set[NUM_SETS];
+};
+struct BlockTables {
+  int S = 0, op_pairs = 0, ldiag = 0;
+  size_t energy, k2, lpref, tcs, ops, cpair;  // offsets into data
+  std::vector<double> data;
+};
+BlockTables block_tables(const BlockModel& m, bool pm);
 hipError_t launch_eval_fp32(int A, int AR, int pm, const EvalArgs& a, hipStream_t s);
 hipError_t launch_eval_batched(int A, int AR, int pm, const LaneProbs& probs, const BatchTile* tiles,
                                int ntiles, int* counter, int waves, hipStream_t s);
