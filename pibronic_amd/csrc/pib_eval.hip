@@ -8,7 +8,7 @@
 // Mapping (gfx950, wave64): G lanes cooperate on one sample, 64/G samples per wave. Lane g
 // owns the contiguous bead chunk [g*K, min((g+1)*K, P)). Per bead it forms the diagonal
 // O-factors of every temperature set, the residual coupling V in registers, M = exp(-tau V)
-// directly (a scaled and squared Taylor polynomial, per lane, A x A in registers; the
+// directly (a scaled and squared polynomial, per lane, A x A in registers; the
 // reference's eigendecomposition serves only to form M) and multiplies M * diag(O_vib / S_p)
 // into its running ring product. The G partial products are
 // then combined by a log2(G)-level ordered tree of A x A products over cross-lane moves
@@ -27,6 +27,7 @@
 #include <type_traits>
 
 #include "pib_common.hpp"
+#include "pib_expm.hpp"
 #include "pib_kernels.hpp"
 
 namespace pib {
@@ -35,20 +36,10 @@ namespace pib {
 // M = exp(X) for a symmetric A x A matrix held in one lane's registers, X = -tau V.
 //
 // The reference forms M = U diag(exp(-tau lambda)) U^T from eigh(V) (pimc.py:1167-1187); M is
-// the only consumer of the decomposition, so it is computed directly: scaling and squaring of
-// a Taylor polynomial, in one of three evaluation schemes (expm_lane picks one per kernel). The
-// first is the degree-12 Taylor polynomial T_12, evaluated by Paterson-Stockmeyer in X^3:
-//   T_12 = ((B3 X^3 + B2) X^3 + B1) X^3 + B0,  B_n = c_3n I + c_3n+1 X + c_3n+2 X^2 (n < 3),
-//   B3 = c9 I + c10 X + c11 X^2 + c12 X^3,
-// five products (X^2, X^3, three Horner steps) against seven for Horner's rule at degree 8.
-// X is scaled by 2^-s so that alpha 2^-s <= theta_12 = 0.2996 (Sastre et al. 2015: the backward
-// error of T_12 below the unit roundoff), alpha = min(|X|_F, |X^3|_F^(1/3)) >= the spectral
-// radius (X^2 and X^3 are formed before scaling; scaling by powers of two is exact). For a
-// symmetric X the 2-norm error of a polynomial in X is its largest error over the eigenvalues.
-// T_12 is then squared s times: on the workload matrices 2.0 squarings per wave at A = 4
-// instead of 5.0 at degree 8 with the Frobenius bound (7.0 instead of 12.0 products per bead).
-// Every intermediate is a polynomial in X, hence symmetric, so products form the upper
-// triangle only. s differs between lanes; the squaring loop runs the wave's largest count.
+// the only consumer of the decomposition, so it is computed directly: scaling and squaring of a
+// polynomial (pib_expm.hpp), in one of two evaluation forms (expm_lane picks one per kernel).
+// Every intermediate is a polynomial in X, hence symmetric, so products form the upper triangle
+// only. s differs between lanes; the squaring loop runs the wave's largest count.
 // Z = X Y + d I for commuting symmetric X, Y (Z symmetric; Z must not alias X or Y)
 template <int A>
 __device__ __forceinline__ void sym_prod_lane(const double (&X)[A][A], const double (&Y)[A][A], double d,
@@ -60,24 +51,6 @@ __device__ __forceinline__ void sym_prod_lane(const double (&X)[A][A], const dou
       double s = (i == k) ? fma(X[i][0], Y[0][k], d) : X[i][0] * Y[0][k];
 #pragma unroll
       for (int c = 1; c < A; ++c) s = fma(X[i][c], Y[c][k], s);
-      Z[i][k] = s;
-      Z[k][i] = s;
-    }
-}
-
-// Z = T Y + c0 I + c1 X + c2 X2 for commuting symmetric T, Y, X, X2 (Z symmetric, no aliasing)
-template <int A>
-__device__ __forceinline__ void sym_prod_add(const double (&T)[A][A], const double (&Y)[A][A], double c0,
-                                             double c1, const double (&X)[A][A], double c2,
-                                             const double (&X2)[A][A], double (&Z)[A][A]) {
-#pragma unroll
-  for (int i = 0; i < A; ++i)
-#pragma unroll
-    for (int k = i; k < A; ++k) {
-      double s = fma(c2, X2[i][k], c1 * X[i][k]);
-      if (i == k) s += c0;
-#pragma unroll
-      for (int c = 0; c < A; ++c) s = fma(T[i][c], Y[c][k], s);
       Z[i][k] = s;
       Z[k][i] = s;
     }
@@ -102,81 +75,15 @@ __device__ __forceinline__ void square_times(double (&T)[A][A], int s) {
   }
 }
 
-constexpr double kLog2Theta12 = -1.738865;  // log2(0.2996)
-
-template <int A>
-__device__ __forceinline__ void expm_lane_ps12(double (&X)[A][A], double (&T)[A][A]) {
-  double X2[A][A], X3[A][A];
-  sym_prod_lane<A>(X, X, 0.0, X2);
-  sym_prod_lane<A>(X2, X, 0.0, X3);
-  double nf = 0.0, n3 = 0.0;
-#pragma unroll
-  for (int i = 0; i < A; ++i) {
-    nf = fma(X[i][i], X[i][i], nf);
-    n3 = fma(X3[i][i], X3[i][i], n3);
-#pragma unroll
-    for (int k = i + 1; k < A; ++k) {
-      nf = fma(2.0 * X[i][k], X[i][k], nf);
-      n3 = fma(2.0 * X3[i][k], X3[i][k], n3);
-    }
-  }
-  const double la = fmin(0.5 * log2_coarse(nf), log2_coarse(n3) / 6.0);
-  const double sd = la - kLog2Theta12;
-  int s = 0;
-  if (sd > 0.0) s = sd < 64.0 ? (int)ceil(sd) : 64;
-#pragma unroll
-  for (int i = 0; i < A; ++i)
-#pragma unroll
-    for (int k = i; k < A; ++k) {
-      X[i][k] = ldexp(X[i][k], -s);
-      X[k][i] = X[i][k];
-      X2[i][k] = ldexp(X2[i][k], -2 * s);
-      X2[k][i] = X2[i][k];
-      X3[i][k] = ldexp(X3[i][k], -3 * s);
-      X3[k][i] = X3[i][k];
-    }
-  constexpr double c[13] = {1.0, 1.0, 1.0 / 2, 1.0 / 6, 1.0 / 24, 1.0 / 120, 1.0 / 720, 1.0 / 5040,
-                            1.0 / 40320, 1.0 / 362880, 1.0 / 3628800, 1.0 / 39916800, 1.0 / 479001600};
-#pragma unroll
-  for (int i = 0; i < A; ++i)
-#pragma unroll
-    for (int k = 0; k < A; ++k) {
-      double v = fma(c[12], X3[i][k], fma(c[11], X2[i][k], c[10] * X[i][k]));
-      T[i][k] = (i == k) ? v + c[9] : v;
-    }
-#pragma unroll
-  for (int n = 2; n >= 0; --n) {
-    double Z[A][A];
-    sym_prod_add<A>(T, X3, c[3 * n], c[3 * n + 1], X, c[3 * n + 2], X2, Z);
-#pragma unroll
-    for (int i = 0; i < A; ++i)
-#pragma unroll
-      for (int k = 0; k < A; ++k) T[i][k] = Z[i][k];
-  }
-  square_times<A>(T, s);
-}
-
-// theta_8 = 0.049: below the root of |y|^8 / 9! = u (the degree-8 polynomial's truncation)
-constexpr double kLog2Theta8 = -4.3511;  // log2(0.049)
-
-// The degree-8 Taylor polynomial with three matrix products (Horner's rule takes seven), in the
-// evaluation form of Sastre (J. Sastre, "Efficient evaluation of matrix polynomials", Linear
-// Algebra Appl. 539 (2018) 229-250):
-//   Y  = X2 (c1 X2 + c2 X),
-//   T8 = (Y + c3 X2 + c4 X)(Y + c5 X2) + c6 Y + X2/2 + X + I,
-// whose coefficients solve the six equations that make the expansion's X^3..X^8 terms 1/k!
-// (c1^2 = 1/8!, 2 c1 c2 = 1/7!, ...; of the two real solution pairs, the one with the smaller
-// c6). Y's product is taken as two dot products per entry (X2 X2 and X2 X), so that no fourth
-// matrix is live beside X, X2 and Y; the three factors of the last product then replace X, X2
-// and Y entry by entry. alpha = |X^2|_F^(1/2), a tighter bound on the spectral radius of a
-// symmetric X than |X|_F (the root of the largest of sum lambda^4), from X2, which the
-// polynomial needs anyway. For |X| <= theta_8 the terms beyond I + X + X^2/2 are below 1e-5 of
-// the result, so the form rounds like Horner's rule.
+// Exp8's degree-8 polynomial in three matrix products (Horner's rule takes seven). Y's product is
+// taken as two dot products per entry (X2 X2 and X2 X) so that no fourth matrix is live beside X,
+// X2 and Y; the three factors of the last product then replace X, X2 and Y entry by entry.
+// alpha = |X^2|_F^(1/2), a tighter bound on the spectral radius of a symmetric X than |X|_F (the
+// root of the largest of sum lambda^4), from X2, which the polynomial needs anyway. The terms
+// beyond I + X + X^2/2 are small against the result, so the form rounds like Horner's rule.
 template <int A>
 __device__ __forceinline__ void expm_lane_s8(double (&X)[A][A], double (&T)[A][A]) {
-  constexpr double c1 = 4.98011920555997349987007158e-3, c2 = 1.99204768222398939994802863e-2;
-  constexpr double c3 = 7.66526532111914669031909419e-2, c4 = 8.76500980178555335977132598e-1;
-  constexpr double c5 = 1.22552115011207473091611921e-1, c6 = 2.97430720484762666375079572e0;
+  using E = Exp8;
   double X2[A][A];
   sym_prod_lane<A>(X, X, 0.0, X2);
   double n2 = 0.0;
@@ -186,8 +93,8 @@ __device__ __forceinline__ void expm_lane_s8(double (&X)[A][A], double (&T)[A][A
 #pragma unroll
     for (int k = i + 1; k < A; ++k) n2 = fma(2.0 * X2[i][k], X2[i][k], n2);
   }
-  // smallest s >= 0 with |X^2|_F^(1/2) 2^-s <= theta_8; a zero matrix gives -inf, NaN s = 0
-  const double sd = 0.25 * log2_coarse(n2) - kLog2Theta8;
+  // smallest s >= 0 with |X^2|_F^(1/2) 2^-s <= theta; a zero matrix gives -inf, NaN s = 0
+  const double sd = 0.25 * log2_coarse(n2) - E::log2_theta;
   int s = 0;
   if (sd > 0.0) s = sd < 64.0 ? (int)ceil(sd) : 64;
 #pragma unroll
@@ -210,20 +117,20 @@ __device__ __forceinline__ void expm_lane_s8(double (&X)[A][A], double (&T)[A][A
         a = fma(X2[i][c], X2[c][k], a);
         b = fma(X2[i][c], X[c][k], b);
       }
-      T[i][k] = fma(c1, a, c2 * b);
+      T[i][k] = fma(E::c1, a, E::c2 * b);
       T[k][i] = T[i][k];
     }
-  // factors in place: X <- Y + c3 X2 + c4 X, X2 <- Y + c5 X2, T <- c6 Y + X2/2 + X + I
+  // factors in place: X <- Y + c3 X2 + c4 X, X2 <- Y + c5 X2, T <- c6 Y + c7 X2 + X + I
 #pragma unroll
   for (int i = 0; i < A; ++i)
 #pragma unroll
     for (int k = i; k < A; ++k) {
       const double x = X[i][k], x2 = X2[i][k], y = T[i][k];
-      double w = fma(c6, y, fma(0.5, x2, x));
+      double w = fma(E::c6, y, fma(E::c7, x2, x));
       if (i == k) w += 1.0;
-      X[i][k] = fma(c3, x2, fma(c4, x, y));
+      X[i][k] = fma(E::c3, x2, fma(E::c4, x, y));
       X[k][i] = X[i][k];
-      X2[i][k] = fma(c5, x2, y);
+      X2[i][k] = fma(E::c5, x2, y);
       X2[k][i] = X2[i][k];
       T[i][k] = w;
       T[k][i] = w;
@@ -242,31 +149,13 @@ __device__ __forceinline__ void expm_lane_s8(double (&X)[A][A], double (&T)[A][A
   square_times<A>(T, s);
 }
 
-// theta_15+ = 0.6764: the largest |X| at which the form below has a relative backward error
-// sum_{k>=16} |h_k| |X|^(k-1) <= 2^-53, h(x) = log(e^-x p(x)) (h_16 = -2.17e-14, h_17 = 1.89e-14)
-constexpr double kLog2Theta15 = -0.5640051;  // log2(0.67642)
-
-// Degree 16 in four products, exact Taylor coefficients through x^15 (x^16 at 0.546 / 16!), in
-// the evaluation form of Sastre (2018) one level up from the degree-8 form:
-//   y02 = X2 (c1 X2 + c2 X),
-//   y12 = (y02 + c3 X2 + c4 X)(y02 + c5 X2) + c6 y02 + c7 X2,
-//   T   = (y12 + c8 X2 + c9 X)(y12 + c10 y02 + c11 X) + c12 y12 + c13 y02 + c14 X2 + X + I.
-// The fourteen coefficients solve the fourteen equations that make the x^2..x^15 terms 1/k! (of
-// the real solutions, one with the smallest coefficients). To keep four matrices live at most, y02
-// is held as G = y02 + c5 X2 (the second factor of y12's product; the later terms in y02 are
-// rewritten in G and X2), and y12's first factor is formed one row at a time. alpha = |X^2|_F^(1/2)
-// as in the degree-8 form; on the A = 8 workload matrices a wave squares 2 times instead of 5-6.
+// Exp16's degree-16 polynomial in four products. To keep four matrices live at most, y02 is held
+// as G = y02 + c5 X2 (the second factor of y12's product; the later terms in y02 are rewritten in G
+// and X2), and y12's first factor is formed one row at a time. alpha as in the degree-8 form; on
+// the A = 4, 6 and 8 workload matrices a wave needs no squaring (Taylor coefficients: 0.5-1.0).
 template <int A>
-__device__ __forceinline__ void expm_lane_s15(double (&X)[A][A], double (&T)[A][A]) {
-  constexpr double c1 = -4.01876161020103546293293287596e-4, c2 = -2.94553144027968298047549126357e-3;
-  constexpr double c3 = 8.70906657683767596765346131523e-3, c4 = -4.01756844067356780152362494573e-1;
-  constexpr double c5 = -3.23076288812231208197540935626e-2, c6 = 2.33731940471157926649827413344e-2;
-  constexpr double c7 = 2.61492797729811710806033238185e-1, c8 = -2.38107037387098722469262858218e-1;
-  constexpr double c9 = -4.1302763659297829110328428344e-2, c10 = -5.79236170707326052179805145605e0;
-  constexpr double c11 = 2.22420917249637356119032703879e0, c12 = 1.04080173523135436461532671084e1;
-  constexpr double c13 = 3.03012340073871230596564458406e0, c14 = -2.12975559049643578453357460382e0;
-  // the same polynomial in G = y02 + c5 X2
-  constexpr double d3 = c3 - c5, e7 = c7 - c6 * c5, f10 = -c10 * c5, g14 = c14 - c13 * c5;
+__device__ __forceinline__ void expm_lane_s16(double (&X)[A][A], double (&T)[A][A]) {
+  using E = Exp16;
   double X2[A][A], Gm[A][A];
   sym_prod_lane<A>(X, X, 0.0, X2);
   double n2 = 0.0;
@@ -276,7 +165,7 @@ __device__ __forceinline__ void expm_lane_s15(double (&X)[A][A], double (&T)[A][
 #pragma unroll
     for (int k = i + 1; k < A; ++k) n2 = fma(2.0 * X2[i][k], X2[i][k], n2);
   }
-  const double sd = 0.25 * log2_coarse(n2) - kLog2Theta15;
+  const double sd = 0.25 * log2_coarse(n2) - E::log2_theta;
   int s = 0;
   if (sd > 0.0) s = sd < 64.0 ? (int)ceil(sd) : 64;
 #pragma unroll
@@ -293,14 +182,14 @@ __device__ __forceinline__ void expm_lane_s15(double (&X)[A][A], double (&T)[A][
   for (int i = 0; i < A; ++i)
 #pragma unroll
     for (int k = i; k < A; ++k) {
-      T[i][k] = fma(c1, X2[i][k], c2 * X[i][k]);
+      T[i][k] = fma(E::c1, X2[i][k], E::c2 * X[i][k]);
       T[k][i] = T[i][k];
     }
 #pragma unroll
   for (int i = 0; i < A; ++i)
 #pragma unroll
     for (int k = i; k < A; ++k) {
-      double acc = c5 * X2[i][k];
+      double acc = E::c5 * X2[i][k];
 #pragma unroll
       for (int c = 0; c < A; ++c) acc = fma(X2[i][c], T[c][k], acc);
       Gm[i][k] = acc;
@@ -311,10 +200,10 @@ __device__ __forceinline__ void expm_lane_s15(double (&X)[A][A], double (&T)[A][
   for (int i = 0; i < A; ++i) {
     double f[A];
 #pragma unroll
-    for (int c = 0; c < A; ++c) f[c] = fma(c4, X[i][c], fma(d3, X2[i][c], Gm[i][c]));
+    for (int c = 0; c < A; ++c) f[c] = fma(E::c4, X[i][c], fma(E::d3, X2[i][c], Gm[i][c]));
 #pragma unroll
     for (int k = i; k < A; ++k) {
-      double acc = fma(c6, Gm[i][k], e7 * X2[i][k]);
+      double acc = fma(E::c6, Gm[i][k], E::e7 * X2[i][k]);
 #pragma unroll
       for (int c = 0; c < A; ++c) acc = fma(f[c], Gm[c][k], acc);
       T[i][k] = acc;
@@ -328,11 +217,11 @@ __device__ __forceinline__ void expm_lane_s15(double (&X)[A][A], double (&T)[A][
 #pragma unroll
     for (int k = i; k < A; ++k) {
       const double x = X[i][k], x2 = X2[i][k], g = Gm[i][k], y = T[i][k];
-      double r = fma(c12, y, fma(c13, g, fma(g14, x2, x)));
+      double r = fma(E::c12, y, fma(E::c13, g, fma(E::g14, x2, x)));
       if (i == k) r += 1.0;
-      X[i][k] = fma(c8, x2, fma(c9, x, y));
+      X[i][k] = fma(E::c8, x2, fma(E::c9, x, y));
       X[k][i] = X[i][k];
-      X2[i][k] = fma(c10, g, fma(c11, x, fma(f10, x2, y)));
+      X2[i][k] = fma(E::c10, g, fma(E::c11, x, fma(E::f10, x2, y)));
       X2[k][i] = X2[i][k];
       T[i][k] = r;
       T[k][i] = r;
@@ -351,21 +240,18 @@ __device__ __forceinline__ void expm_lane_s15(double (&X)[A][A], double (&T)[A][
   square_times<A>(T, s);
 }
 
-// Which scheme each kernel uses: the four-product degree-15+ form without +-dbeta (its four
-// live matrices fit beside one ring state), except at A = 6, whose kernel holds two waves per
-// SIMD in 256 VGPRs and spills with four live matrices; else Paterson-Stockmeyer degree 12 for
-// A <= 4 and the three-product degree-8 form above (the +-dbeta kernels carry three ring states).
-// Measured on MI355X (eval ms, degree 15+ against the previous scheme, 1e5 samples, same GPU):
-// A=4 N=8 P=64 0.308 / 0.315 (PS-12), A=5 N=10 P=64 0.472 / 0.508, A=6 N=12 P=128 1.758 / 1.427
-// (spilling), A=7 N=14 P=64 1.173 / 1.260, A=8 N=16 P=64 1.723 / 1.846 (4.05 / 4.43 at 262,144).
+// Which form each kernel uses: four products at degree 16, except at A = 6 without +-dbeta, whose
+// kernel holds two waves per SIMD in 256 VGPRs and spills with four live matrices: degree 8 in
+// three products there. Measured on MI355X (eval us, 1e5 samples, P = 64, N = 2 A; Taylor
+// polynomials of the same forms / these): A = 4 282 / 271, A = 7 1214 / 1177; A = 6 at P = 128
+// 1352 / 1294; with +-dbeta A = 4 437 (degree 12 in five products) / 408, A = 5 942 / 906 and A = 6
+// 1454 / 1387 (degree 8).
 template <int A, bool PM>
 __device__ __forceinline__ void expm_lane(double (&X)[A][A], double (&T)[A][A]) {
-  if constexpr (!PM && A != 6)
-    expm_lane_s15<A>(X, T);
-  else if constexpr (A <= 4)
-    expm_lane_ps12<A>(X, T);
-  else
+  if constexpr (!PM && A == 6)
     expm_lane_s8<A>(X, T);
+  else
+    expm_lane_s16<A>(X, T);
 }
 
 template <int A, int AR, bool PM, bool QD, class Q>
@@ -622,7 +508,6 @@ __device__ __forceinline__ void eval_wave(const EvalArgs& args, int64_t wave) {
       }
     }
   }
-
 
   // ordered tree over the G lanes of a sample: lane g (g % 2s == 0) absorbs lane g + s
   for (int s = 1; s < G; s <<= 1) {

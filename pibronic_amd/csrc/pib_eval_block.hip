@@ -18,17 +18,17 @@
 //    matrix elements (or surfaces) as rows and four modes per instruction; the coefficient
 //    operands come from a table laid out in operand order. X = -tau V is handed to the
 //    4 x 4 layout through LDS (lower triangles; the reads mirror them).
-//  * back: step by step, M = exp(X) by the scaled and squared degree-15+ form of the per-lane
+//  * back: step by step, M = exp(X) by the scaled and squared degree-16 form of the per-lane
 //    kernel, and the ring products R^T <- diag(O / S) M R^T of every chain (one, or three with
 //    +-dbeta).
 // Padding: rows and columns >= A of X are zero and the Taylor identity covers only the leading
 // A x A block, so M is zero outside it; padded surfaces have log F = -inf, O = 0.
 //
-// Measured (MI355X, evaluation of 1e5 samples at A = 8, N = 16, P = 64, us): 1416 against 1650 for the
+// Measured (MI355X, evaluation of 1e5 samples at A = 8, N = 16, P = 64, us): 1327 against 1650 for the
 // per-lane kernel (one wave per SIMD, a third of its vector instructions moves to and from the
-// accumulation registers); with +-dbeta 1882 against 5470 for three single-chain passes of that
+// accumulation registers); with +-dbeta 1793 against 5470 for three single-chain passes of that
 // kernel. With +-dbeta at A = 12, N = 24, P = 128, 16,384 samples 1478 against 5720 for the
-// one-wave-per-sample kernel; at A = 11, N = 17, P = 50, 3,001 samples 128 against 373.
+// one-wave-per-sample kernel; at A = 11, N = 17, P = 50, 3,001 samples 122 against 373.
 //
 // What bounds it: FP64 issue. On gfx950 the FP64 matrix and vector instructions share one pipe
 // (timed together they add up exactly: 8 mfma_f64_4x4x4 + 32 v_fma_f64 take 311 cycles per SIMD,
@@ -36,6 +36,7 @@
 // instructions are the cheaper ones (18.8 cycles per 4x4x4x4, 70 per 16x16x4, 5.4 per v_fma_f64).
 #include "pib_common.hpp"
 #include "pib_ctx.hpp"
+#include "pib_expm.hpp"
 #include "pib_kernels.hpp"
 
 namespace pib {
@@ -114,8 +115,6 @@ __device__ __forceinline__ double down(double c, int k) {
   return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | (unsigned)u);
 }
 
-constexpr double kLog2Theta15 = -0.5640051;  // log2(0.67642)
-
 // Z = X Y + Z for commuting symmetric X, Y and a symmetric Z given by its blocks I <= K
 template <int NB>
 __device__ __forceinline__ void sym_mul_upper(const double (&X)[NB][NB], const double (&Y)[NB][NB],
@@ -146,22 +145,14 @@ __device__ __forceinline__ void sym_mul(const double (&X)[NB][NB], const double 
   mirror<NB>(Z, ident);
 }
 
-// T = exp(X) of the wave's four symmetric matrices, zero outside the leading n x n block: the
-// four-product degree-15+ form of the per-lane kernel (after Sastre 2018; pib_eval.hip gives the
-// form, its coefficients' defining equations and theta). One squaring count for the four
+// T = exp(X) of the wave's four symmetric matrices, zero outside the leading n x n block: Exp16's
+// degree-16 polynomial in four products, scaled and squared. One squaring count for the four
 // matrices, so the scaling by 2^-s goes into the (scalar) coefficients instead of X and X^2.
 // alpha = |X^2|_F^(1/2) needs only its binary exponent: its sum is taken in FP32.
 template <int NB>
 __device__ __forceinline__ void expm_block(const double (&X)[NB][NB], int n, int i, int j, double ident,
                                            double (&T)[NB][NB]) {
-  constexpr double c1 = -4.01876161020103546293293287596e-4, c2 = -2.94553144027968298047549126357e-3;
-  constexpr double c3 = 8.70906657683767596765346131523e-3, c4 = -4.01756844067356780152362494573e-1;
-  constexpr double c5 = -3.23076288812231208197540935626e-2, c6 = 2.33731940471157926649827413344e-2;
-  constexpr double c7 = 2.61492797729811710806033238185e-1, c8 = -2.38107037387098722469262858218e-1;
-  constexpr double c9 = -4.1302763659297829110328428344e-2, c10 = -5.79236170707326052179805145605e0;
-  constexpr double c11 = 2.22420917249637356119032703879e0, c12 = 1.04080173523135436461532671084e1;
-  constexpr double c13 = 3.03012340073871230596564458406e0, c14 = -2.12975559049643578453357460382e0;
-  constexpr double d3 = c3 - c5, e7 = c7 - c6 * c5, f10 = -c10 * c5, g14 = c14 - c13 * c5;
+  using E = Exp16;
   double X2[NB][NB], G[NB][NB], F[NB][NB];
   sym_mul<NB>(X, X, ident, X2);
   double nd = 0.0, no = 0.0;
@@ -185,12 +176,12 @@ __device__ __forceinline__ void expm_block(const double (&X)[NB][NB], int n, int
   m = fmaxf(m, dpp_f<0x124>(m));  // the largest of the four streams: row_ror 4, 8
   m = fmaxf(m, dpp_f<0x128>(m));
   // smallest s >= 0 with alpha 2^-s <= theta; a zero matrix gives -inf, a NaN s = 0
-  const float sd = 0.25f * __log2f(m) - (float)kLog2Theta15;
+  const float sd = 0.25f * __log2f(m) - (float)E::log2_theta;
   int s = 0;
   if (sd > 0.0f) s = sd < 64.0f ? (int)ceilf(sd) : 64;
   s = __builtin_amdgcn_readfirstlane(s);
   {
-    const double k1 = down(c1, 4 * s), k2 = down(c2, 3 * s), k5 = down(c5, 2 * s);
+    const double k1 = down(E::c1, 4 * s), k2 = down(E::c2, 3 * s), k5 = down(E::c5, 2 * s);
 #pragma unroll
     for (int I = 0; I < NB; ++I)
 #pragma unroll
@@ -202,29 +193,29 @@ __device__ __forceinline__ void expm_block(const double (&X)[NB][NB], int n, int
   sym_mul_upper<NB>(X2, F, G);  // G = y02 + c5 X2
   mirror<NB>(G, ident);
   {
-    const double k3 = down(d3, 2 * s), k4 = down(c4, s), k7 = down(e7, 2 * s);
+    const double k3 = down(E::d3, 2 * s), k4 = down(E::c4, s), k7 = down(E::e7, 2 * s);
 #pragma unroll
     for (int I = 0; I < NB; ++I)
 #pragma unroll
       for (int K = 0; K < NB; ++K) {
         F[I][K] = fma(k4, X[I][K], fma(k3, X2[I][K], G[I][K]));
-        if (K >= I) T[I][K] = fma(c6, G[I][K], k7 * X2[I][K]);
+        if (K >= I) T[I][K] = fma(E::c6, G[I][K], k7 * X2[I][K]);
       }
   }
   sym_mul_upper<NB>(F, G, T);  // T = y12
   mirror<NB>(T, ident);
   {
-    const double k8 = down(c8, 2 * s), k9 = down(c9, s), k11 = down(c11, s), k10 = down(f10, 2 * s);
-    const double k14 = down(g14, 2 * s), kx = down(1.0, s);
+    const double k8 = down(E::c8, 2 * s), k9 = down(E::c9, s), k11 = down(E::c11, s), k10 = down(E::f10, 2 * s);
+    const double k14 = down(E::g14, 2 * s), kx = down(1.0, s);
 #pragma unroll
     for (int I = 0; I < NB; ++I)
 #pragma unroll
       for (int K = 0; K < NB; ++K) {
         const double x = X[I][K], x2 = X2[I][K], gg = G[I][K], y = T[I][K];
         F[I][K] = fma(k8, x2, fma(k9, x, y));
-        G[I][K] = fma(c10, gg, fma(k11, x, fma(k10, x2, y)));
+        G[I][K] = fma(E::c10, gg, fma(k11, x, fma(k10, x2, y)));
         if (K >= I) {
-          double r = fma(c12, y, fma(c13, gg, fma(k14, x2, kx * x)));
+          double r = fma(E::c12, y, fma(E::c13, gg, fma(k14, x2, kx * x)));
           if (K == I) r += (i == j && 4 * I + i < n) ? 1.0 : 0.0;
           T[I][K] = r;
         }
