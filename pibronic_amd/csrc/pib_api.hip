@@ -59,6 +59,12 @@ int rebuild_mode_table(pib_ctx* c) {
       }
     }
   }
+  // rho is usually the coupled model's own surface diagonal, and folding leaves no diagonal in the
+  // linear couplings: the lanes kernels then form each O-exponent once and skip those products
+  c->fold = AR == A && c->h_th[SET_RHO] == c->h_th[SET_VIB] && c->h_cs[SET_RHO] == c->h_cs[SET_VIB] &&
+            c->h_lin[SET_RHO] == c->h_lin[SET_VIB] && c->h_k2[SET_RHO] == c->h_k2[SET_VIB];
+  for (int j = 0; j < N && c->fold; ++j)
+    for (int b = 0; b < A; ++b) c->fold = c->fold && c->h_linear[(size_t)j * AA + b * A + b] == 0.0;
   // float copy, records padded to 16 bytes (and zero records up to N4, as above)
   std::vector<float> tabf((size_t)N4 * R.len_f(), 0.f);
   for (int j = 0; j < N; ++j)
@@ -226,6 +232,7 @@ int make_eval_args(pib_ctx* c, int flags, int64_t B, EvalArgs* out_args, bool* w
   a.G = c->lanes ? c->lanes : auto_lanes(c, B, fp32);
   a.K = (c->P + a.G - 1) / a.G;
   a.noscale = (flags & PIB_EVAL_NOSCALE) ? 1 : 0;
+  a.fold = c->fold;
   a.tau = c->tau;
   for (int s = 0; s < NUM_SETS; ++s) {
     a.set[s].coth = (const double*)c->coth[s].p;

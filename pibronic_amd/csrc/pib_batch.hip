@@ -130,7 +130,11 @@ int build_schedule(pib_batch* b) {
   std::stable_sort(tiles.begin(), tiles.end(), [](const T& x, const T& y) { return x.cost > y.cost; });
   if (b->lane_ok) {
     b->lprobs.n = b->n;
-    for (int i = 0; i < b->n; ++i) b->lprobs.p[i] = lane_prob(b->args[i]);
+    b->lprobs.fold = 1;
+    for (int i = 0; i < b->n; ++i) {
+      b->lprobs.p[i] = lane_prob(b->args[i]);
+      b->lprobs.fold = b->lprobs.fold && b->args[i].fold;
+    }
   }
   std::vector<BatchTile> ht(tiles.size());
   for (size_t k = 0; k < tiles.size(); ++k) ht[k] = tiles[k].t;

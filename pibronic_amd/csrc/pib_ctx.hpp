@@ -42,6 +42,7 @@ struct pib_ctx {
   std::vector<double> h_linear, h_qdiag;
   pib::DevBuf mode_tab, mode_tab_f, k2_f[pib::NUM_SETS];
   bool mode_tab_ok = false;
+  bool fold = false;  // EvalArgs.fold
   // block kernel: its constants (block_tables) and the host copies they are built from
   std::vector<double> h_energy, h_qpair, h_k2[pib::NUM_SETS], h_lpref[pib::NUM_SETS];
   std::vector<int> h_pairs;

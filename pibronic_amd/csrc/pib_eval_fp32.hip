@@ -125,7 +125,8 @@ __device__ __forceinline__ void expm_lane_f(float (&X)[A][A], float (&T)[A][A]) 
   }
 }
 
-template <int A, int AR, bool PM, bool QD>
+// FOLD: as in the FP64 kernel (mode_terms in pib_eval.hip)
+template <int A, int AR, bool PM, bool QD, bool FOLD>
 __device__ __forceinline__ void mode_terms_f(const float* __restrict__ tab, const CoordBuf& qs, int N, int P,
                                              int p, int pn, float& tr, float& tv, float& tp, float& tm,
                                              float (&er)[AR], float (&ev)[A], float (&ep)[A], float (&em)[A],
@@ -136,14 +137,15 @@ __device__ __forceinline__ void mode_terms_f(const float* __restrict__ tab, cons
     const float x0 = (float)x0d, xn = (float)xnd;
     const float sx = x0 + xn, dx = x0 - xn;
     const float q2s = fmaf(x0, x0, xn * xn), d2 = dx * dx;
-    tr = fmaf(t[1], d2, fmaf(t[0], q2s, tr));
+    if (!FOLD) tr = fmaf(t[1], d2, fmaf(t[0], q2s, tr));
     tv = fmaf(t[3], d2, fmaf(t[2], q2s, tv));
     if (PM) {
       tp = fmaf(t[R.pm() + 1], d2, fmaf(t[R.pm() + 0], q2s, tp));
       tm = fmaf(t[R.pm() + 3], d2, fmaf(t[R.pm() + 2], q2s, tm));
     }
 #pragma unroll
-    for (int a = 0; a < AR; ++a) er[a] = fmaf(t[R.lin_rho() + a], sx, er[a]);
+    for (int a = 0; a < AR; ++a)
+      if (!FOLD) er[a] = fmaf(t[R.lin_rho() + a], sx, er[a]);
 #pragma unroll
     for (int a = 0; a < A; ++a) {
       ev[a] = fmaf(t[R.lin_vib() + a], sx, ev[a]);
@@ -157,7 +159,7 @@ __device__ __forceinline__ void mode_terms_f(const float* __restrict__ tab, cons
     for (int b = 0, e = 0; b < A; ++b)
 #pragma unroll
       for (int c = 0; c <= b; ++c, ++e) {
-        v[b][c] = fmaf(t[R.lin_q() + e], x0, v[b][c]);
+        if (!FOLD || c < b) v[b][c] = fmaf(t[R.lin_q() + e], x0, v[b][c]);
         if (QD) v[b][c] = fmaf(t[R.quad() + e], xx, v[b][c]);
       }
   };
@@ -232,7 +234,7 @@ __device__ __forceinline__ float shfl_down_f(float v, int d) { return __shfl_dow
 
 }  // namespace
 
-template <int A, int AR, bool PM>
+template <int A, int AR, bool PM, bool FOLD = false>
 __global__ void __launch_bounds__(256) k_eval_fp32(const EvalArgs args) {
   const int lane = threadIdx.x & (kWave - 1);
   const int64_t wave = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kWave;
@@ -280,9 +282,9 @@ __global__ void __launch_bounds__(256) k_eval_fp32(const EvalArgs args) {
       for (int c = 0; c <= a; ++c) v[a][c] = 0.0f;
     }
     if (has_q)
-      mode_terms_f<A, AR, PM, true>(args.mode_tab_f, qb, N, P, p, pn, tr, tv, tpl, tmi, er, ev, epl, emi, v);
+      mode_terms_f<A, AR, PM, true, FOLD>(args.mode_tab_f, qb, N, P, p, pn, tr, tv, tpl, tmi, er, ev, epl, emi, v);
     else
-      mode_terms_f<A, AR, PM, false>(args.mode_tab_f, qb, N, P, p, pn, tr, tv, tpl, tmi, er, ev, epl, emi, v);
+      mode_terms_f<A, AR, PM, false, FOLD>(args.mode_tab_f, qb, N, P, p, pn, tr, tv, tpl, tmi, er, ev, epl, emi, v);
     for (int t = 0; t < args.npair; ++t) {
       const int jj = args.pair[2 * t], kk = args.pair[2 * t + 1];
       const float xj = (float)qs[jj * P + p], xk = (float)qs[kk * P + p];
@@ -298,7 +300,10 @@ __global__ void __launch_bounds__(256) k_eval_fp32(const EvalArgs args) {
     float lS = -INFINITY;
 #pragma unroll
     for (int a = 0; a < AR; ++a) {
-      lOr[a] = fmaf(-0.5f, (tr + er[a]) + fr.k2[a], fr.lpref[a]);
+      if constexpr (FOLD)
+        lOr[a] = fmaf(-0.5f, (tv + ev[a]) + fv.k2[a], fr.lpref[a]);
+      else
+        lOr[a] = fmaf(-0.5f, (tr + er[a]) + fr.k2[a], fr.lpref[a]);
       lS = fmaxf(lS, lOr[a]);
     }
 #pragma unroll
@@ -428,8 +433,13 @@ static hipError_t launch_f(int pm, const EvalArgs& a, hipStream_t s) {
   const int spw = kWave / a.G;
   const int64_t waves = (a.B + spw - 1) / spw;
   const dim3 grid((unsigned)((waves * kWave + 255) / 256));
-  if (pm)
+  const bool fold = A == AR && a.fold;
+  if (pm && fold)
+    hipLaunchKernelGGL((k_eval_fp32<A, AR, true, A == AR>), grid, dim3(256), 0, s, a);
+  else if (pm)
     hipLaunchKernelGGL((k_eval_fp32<A, AR, true>), grid, dim3(256), 0, s, a);
+  else if (fold)
+    hipLaunchKernelGGL((k_eval_fp32<A, AR, false, A == AR>), grid, dim3(256), 0, s, a);
   else
     hipLaunchKernelGGL((k_eval_fp32<A, AR, false>), grid, dim3(256), 0, s, a);
   return hipGetLastError();

@@ -50,6 +50,8 @@ struct EvalArgs {
   int G;                // lanes per sample (power of two, divides 64)
   int K;                // beads per lane = ceil(P / G)
   int noscale;          // 1: skip the S12 scaling (S_p = 1), as the reference's explicit test
+  int fold;             // rho's O-exponent constants (th, csch, lin, k2) equal vib's bit for bit, and
+                        // every linear coupling's diagonal is zero (see mode_terms)
   double tau;           // M-matrix step (always the base tau, quirk Q1)
   OSet set[NUM_SETS];
   const double* energy;   // A*A, diagonal zeroed
@@ -160,6 +162,7 @@ struct LaneProb {
 };
 struct LaneProbs {
   int n;
+  int fold;  // every problem's EvalArgs.fold
   LaneProb p[kBatchLaunchProbs];
 };
 
