@@ -1028,8 +1028,10 @@ int pib_flow_logrho(pib_ctx* c, int64_t B, const double* R, const double* cb, fl
   if (B < 0 || !R || (!dR && !logrho)) return fail(c, PIB_ERR_ARG, "flow_logrho: B < 0 or nothing to compute");
   LogRhoArgs a{};
   a.B = B; a.N = c->set_N[SET_RHO]; a.P = c->P; a.A = c->set_A[SET_RHO];
-  a.coth = (const double*)c->coth[SET_RHO].p;
+  a.th = (const double*)c->th[SET_RHO].p;
   a.csch = (const double*)c->csch[SET_RHO].p;
+  a.lin = (const double*)c->lin[SET_RHO].p;
+  a.k2 = (const double*)c->k2[SET_RHO].p;
   a.pref = (const double*)c->pref[SET_RHO].p;
   a.shift = (const double*)c->shift[SET_RHO].p;
   a.R = R; a.c = cb; a.dR = dR; a.logrho = logrho;

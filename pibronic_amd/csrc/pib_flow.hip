@@ -497,70 +497,78 @@ hipError_t launch_coupling_inverse_backward(const CouplingArgs& a, hipStream_t s
 
 // ------------------------------------------------------------------ log rho and its gradient
 // rho(R) = sum_a prod_p O^rho_a(p) of the sampling model (pibronic/pimc/pimc.py:1087-1136,
-// unscaled), log_a = P log F_a - 1/2 sum_jp [coth_j (x_p^2 + x_{p+1}^2) - 2 csch_j x_p x_{p+1}],
-// x = R - d_a. d log_a / dx_p = -(2 coth_j x_p - csch_j (x_{p-1} + x_{p+1})). The gradient of
-// log rho is the responsibility-weighted sum over surfaces. One work-group per sample.
+// unscaled). Summed over the ring, the expanded exponent of the evaluation kernels (OSet) needs the
+// surfaces only through the coordinates' sums:
+//   log_a = P log F_a - 1/2 [sum_jp th_j (x_p^2 + x_{p+1}^2) + csch_j (x_p - x_{p+1})^2
+//                            + 2 sum_j lin_aj sum_p x_jp + P k2_a],
+// so a coordinate costs 5 + A operations instead of 7 A, without the cancellation of
+// coth (x1^2 + x2^2) - 2 csch x1 x2. With the responsibilities' mean displacement
+// m_j = sum_a resp_a d_aj the gradient of log rho is
+//   -(2 coth_j x_p - csch_j (x_{p-1} + x_{p+1}) - 2 th_j m_j).
+// One wave per sample. Measured (MI355X, us, 7 A operations per coordinate and a log and an exp per
+// surface / this): 32,768 samples at A = 4, N = 8, P = 64 90 / 47, 131,072 at A = 8, N = 16, P = 64
+// 761 / 402, 2,048 there with the gradient 48 / 22. Reading takes 28 us of the 47; the rest is the
+// A + 2 sums over the wave and the transcendental tail of each sample.
 constexpr int kMaxRhoSurfaces = 16;
 
+template <int MAXA>
 __global__ void __launch_bounds__(64 * kRowsPerBlock) k_logrho(LogRhoArgs a) {
   const int lane = threadIdx.x & 63;
   const int64_t b = (int64_t)blockIdx.x * kRowsPerBlock + threadIdx.x / 64;
   if (b >= a.B) return;  // whole wave
   const int N = a.N, P = a.P, NP = N * P;
-  const double* R = a.R + b * (int64_t)NP;
-  double part[kMaxRhoSurfaces];
+  const double* __restrict__ R = a.R + b * (int64_t)NP;
+  // mode-uniform constants by scalar loads
+  const auto th = as_const(a.th), cs = as_const(a.csch), lin = as_const(a.lin), shift = as_const(a.shift);
+  double t = 0.0, part[MAXA];
 #pragma unroll
-  for (int s = 0; s < kMaxRhoSurfaces; ++s) part[s] = 0.0;
-  for (int j = 0; j < N; ++j) {  // mode-uniform constants: scalar loads, no index division
-    const double cj = a.coth[j], sj2 = 2.0 * a.csch[j];
-    for (int p = lane; p < P; p += 64) {
-      const int pn = (p + 1 == P) ? 0 : p + 1;
-      const double r0 = R[j * P + p], r1 = R[j * P + pn];
+  for (int s = 0; s < MAXA; ++s) part[s] = 0.0;
+  for (int p = lane; p < P; p += 64) {
+    const int pn = (p + 1 == P) ? 0 : p + 1;
+#pragma unroll 4
+    for (int j = 0; j < N; ++j) {
+      const double x = R[j * P + p], xn = R[j * P + pn];
+      const double d = x - xn;
+      t = fma(cs[j], d * d, fma(th[j], fma(x, x, xn * xn), t));
 #pragma unroll
-      for (int s = 0; s < kMaxRhoSurfaces; ++s) {
-        if (s < a.A) {
-          const double d = a.shift[s * N + j];
-          const double x1 = r0 - d, x2 = r1 - d;
-          part[s] += cj * (x1 * x1 + x2 * x2) - (sj2 * x1) * x2;
-        }
-      }
+      for (int s = 0; s < MAXA; ++s)
+        if (s < a.A) part[s] = fma(lin[s * N + j], x, part[s]);
     }
   }
-  // every lane ends with the same sums (xor butterfly), so every lane holds la, lmax, tot
-  double lmax = -INFINITY;
-  double la[kMaxRhoSurfaces];
+  // lane s finishes surface s, so that the wave takes one log and one exp for all of them
+  t = wave_sum_d(t);
+  double la = -INFINITY;
 #pragma unroll
-  for (int s = 0; s < kMaxRhoSurfaces; ++s) {
-    la[s] = -INFINITY;
+  for (int s = 0; s < MAXA; ++s)
     if (s < a.A) {
-      la[s] = P * log(a.pref[s]) - 0.5 * wave_sum_d(part[s]);
-      lmax = fmax(lmax, la[s]);
+      const double v = wave_sum_d(part[s]);
+      la = lane == s ? v : la;
     }
-  }
-  double tot = 0.0;
+  if (lane < a.A) la = P * log(a.pref[lane]) - 0.5 * (t + fma(2.0, la, P * a.k2[lane]));
+  double lmax = la;
 #pragma unroll
-  for (int s = 0; s < kMaxRhoSurfaces; ++s)
-    if (s < a.A) tot += exp(la[s] - lmax);
+  for (int m = 1; m < 16; m *= 2) lmax = fmax(lmax, __shfl_xor(lmax, m, 16));
+  lmax = __shfl(lmax, 0, 64);
+  const double e = lane < a.A ? exp(la - lmax) : 0.0;
+  const double tot = wave_sum_d(e);
   if (lane == 0 && a.logrho) a.logrho[b] = lmax + log(tot);
   if (!a.dR) return;
-  double resp[kMaxRhoSurfaces];
+  const double cb = a.c ? a.c[b] : 1.0, r = e / tot;
+  double resp[MAXA];
 #pragma unroll
-  for (int s = 0; s < kMaxRhoSurfaces; ++s) resp[s] = (s < a.A) ? exp(la[s] - lmax) / tot : 0.0;
-  const double cb = a.c ? a.c[b] : 1.0;
-  for (int j = 0; j < N; ++j) {
-    const double cj2 = 2.0 * a.coth[j], sj = a.csch[j];
-    for (int p = lane; p < P; p += 64) {
-      const int pn = (p + 1 == P) ? 0 : p + 1, pp = (p == 0) ? P - 1 : p - 1;
-      const double r0 = R[j * P + p], rn = R[j * P + pn], rp = R[j * P + pp];
-      double g = 0.0;
+  for (int s = 0; s < MAXA; ++s) resp[s] = __shfl(r, s, 64);
+  float* __restrict__ dR = a.dR + b * (int64_t)NP;
+  for (int p = lane; p < P; p += 64) {
+    const int pn = (p + 1 == P) ? 0 : p + 1, pp = (p == 0) ? P - 1 : p - 1;
+#pragma unroll 4
+    for (int j = 0; j < N; ++j) {
+      double m = 0.0;
 #pragma unroll
-      for (int s = 0; s < kMaxRhoSurfaces; ++s) {
-        if (s < a.A) {
-          const double d = a.shift[s * N + j];
-          g -= resp[s] * (cj2 * (r0 - d) - sj * ((rn - d) + (rp - d)));
-        }
-      }
-      a.dR[b * (int64_t)NP + j * P + p] = (float)(-cb * g);
+      for (int s = 0; s < MAXA; ++s)
+        if (s < a.A) m = fma(resp[s], shift[s * N + j], m);
+      const double thj = th[j], sj = cs[j];
+      const double g = fma(2.0 * (thj + sj), R[j * P + p], -fma(sj, R[j * P + pn] + R[j * P + pp], 2.0 * thj * m));
+      dR[j * P + p] = (float)(cb * g);
     }
   }
 }
@@ -568,8 +576,13 @@ __global__ void __launch_bounds__(64 * kRowsPerBlock) k_logrho(LogRhoArgs a) {
 hipError_t launch_logrho(const LogRhoArgs& a, hipStream_t s) {
   if (a.A > kMaxRhoSurfaces) return hipErrorInvalidValue;
   if (a.B < 1) return hipSuccess;
-  hipLaunchKernelGGL(k_logrho, dim3((unsigned)((a.B + kRowsPerBlock - 1) / kRowsPerBlock)),
-                     dim3(64 * kRowsPerBlock), 0, s, a);
+  const dim3 grid((unsigned)((a.B + kRowsPerBlock - 1) / kRowsPerBlock)), block(64 * kRowsPerBlock);
+  if (a.A <= 4)
+    hipLaunchKernelGGL(k_logrho<4>, grid, block, 0, s, a);
+  else if (a.A <= 8)
+    hipLaunchKernelGGL(k_logrho<8>, grid, block, 0, s, a);
+  else
+    hipLaunchKernelGGL(k_logrho<16>, grid, block, 0, s, a);
   return hipGetLastError();
 }
 

@@ -131,8 +131,10 @@ hipError_t launch_coupling_inverse_backward(const CouplingArgs& a, hipStream_t s
 struct LogRhoArgs {
   int64_t B;
   int N, P, A;            // A = sampling-model surfaces
-  const double* coth;     // N
+  const double* th;       // N, coth - csch (as OSet)
   const double* csch;     // N
+  const double* lin;      // A * N
+  const double* k2;       // A
   const double* pref;     // A
   const double* shift;    // A * N
   const double* R;        // (B, N, P)
