@@ -99,11 +99,13 @@ void drop_graph(pib_batch* b) {
 // Tiles of `tile_waves` waves (lanes family) or samples (wide family), ordered by decreasing
 // estimated cost so that the longest tiles start first.
 int build_schedule(pib_batch* b) {
-  struct T {
-    BatchTile t;
+  struct Group {  // tiles of one problem and one size
+    int prob, nwaves;
+    int64_t wave0, ntiles;
     double cost;
   };
-  std::vector<T> tiles;
+  std::vector<Group> groups;
+  size_t ntiles = 0;
   for (int i = 0; i < b->n; ++i) {
     EvalArgs& a = b->args[i];
     int64_t units;
@@ -118,16 +120,13 @@ int build_schedule(pib_batch* b) {
       units = b->B;
       unit_cost = (double)a.P;
     }
-    for (int64_t w = 0; w < units; w += b->tile_waves) {
-      T t;
-      t.t.prob = i;
-      t.t.wave0 = w;
-      t.t.nwaves = (int)std::min<int64_t>(b->tile_waves, units - w);
-      t.cost = unit_cost * t.t.nwaves;
-      tiles.push_back(t);
-    }
+    const int64_t full = units / b->tile_waves;
+    const int rest = (int)(units - full * b->tile_waves);
+    if (full) groups.push_back({i, b->tile_waves, 0, full, unit_cost * b->tile_waves});
+    if (rest) groups.push_back({i, rest, full * b->tile_waves, 1, unit_cost * rest});
+    ntiles += full + (rest != 0);
   }
-  std::stable_sort(tiles.begin(), tiles.end(), [](const T& x, const T& y) { return x.cost > y.cost; });
+  std::stable_sort(groups.begin(), groups.end(), [](const Group& x, const Group& y) { return x.cost > y.cost; });
   if (b->lane_ok) {
     b->lprobs.n = b->n;
     b->lprobs.fold = 1;
@@ -136,9 +135,17 @@ int build_schedule(pib_batch* b) {
       b->lprobs.fold = b->lprobs.fold && b->args[i].fold;
     }
   }
-  std::vector<BatchTile> ht(tiles.size());
-  for (size_t k = 0; k < tiles.size(); ++k) ht[k] = tiles[k].t;
-  if (ht.size() > (size_t)0x7fffffff) return bfail(b, PIB_ERR_ARG, "batch: too many tiles");
+  if (ntiles > (size_t)0x7fffffff) return bfail(b, PIB_ERR_ARG, "batch: too many tiles");
+  std::vector<BatchTile> ht;
+  ht.reserve(ntiles);
+  for (const Group& g : groups)
+    for (int64_t k = 0; k < g.ntiles; ++k) {
+      BatchTile t;
+      t.prob = g.prob;
+      t.wave0 = g.wave0 + k * g.nwaves;
+      t.nwaves = g.nwaves;
+      ht.push_back(t);
+    }
   b->ntiles = (int)ht.size();
   PIB_BHIP(b, hipDeviceSynchronize());  // no queued launch may still read the old schedule
   release(b->d_tiles);
@@ -225,6 +232,14 @@ SumArgs sum_args(pib_batch* b, int i, const int64_t* step) {
   return a;
 }
 
+// all problems' samplers, longest rows first
+std::vector<SampleArgs> sampler_args(pib_batch* b, uint64_t seed, const int64_t* step) {
+  std::vector<SampleArgs> v;
+  for (int i = 0; i < b->n; ++i) v.push_back(sample_args(b, i, seed, step));
+  std::stable_sort(v.begin(), v.end(), [](const SampleArgs& x, const SampleArgs& y) { return x.P > y.P; });
+  return v;
+}
+
 double time_ms(pib_batch* b, hipStream_t s, int reps, int* rc) {
   hipEvent_t e0, e1;
   *rc = PIB_OK;
@@ -309,7 +324,7 @@ int pib_batch_create(int n, pib_ctx* const* ctxs, int64_t B, int flags, double d
   if ((r = balloc(b, b->d_args, (size_t)n * sizeof(EvalArgs)))) return r;
   if ((r = balloc(b, b->d_counter, sizeof(int)))) return r;
   if ((r = balloc(b, b->d_step, sizeof(int64_t)))) return r;
-  if ((r = balloc(b, b->partials, (size_t)b->nparts * NUM_SUMS * sizeof(double)))) return r;
+  if ((r = balloc(b, b->partials, (size_t)n * b->nparts * NUM_SUMS * sizeof(double)))) return r;
   b->bound.assign(n, false);
   for (int i = 0; i < n; ++i) {
     b->args[i].q = nullptr;
@@ -324,7 +339,11 @@ int pib_batch_create(int n, pib_ctx* const* ctxs, int64_t B, int flags, double d
               : b->lane_ok            ? PIB_BATCH_LANES
               : b->wide_ok            ? PIB_BATCH_WIDE
                                       : PIB_BATCH_SEQUENTIAL;
-  b->tile_waves = 4;
+  // the persistent lanes kernel's problems share the chip: as many waves as one block of all their
+  // samples needs
+  if (b->family == PIB_BATCH_LANES)
+    for (int i = 0; i < n; ++i) b->lanes[i] = auto_lanes(ctxs[i], B * n, false, true);
+  b->tile_waves = b->family == PIB_BATCH_LANES ? 1 : 4;
   b->grid_waves = b->num_cu * 8;
   PIB_BHIP(b, hipStreamCreateWithFlags(&b->cap, hipStreamNonBlocking));
   return build_schedule(b);
@@ -434,7 +453,7 @@ int pib_batch_tune(pib_batch* b, uint64_t seed, double* best_ms, double* sequent
   int rc0 = check_bound(b, "batch_tune");
   if (!rc0) rc0 = check_samplers(b, "batch_tune");
   if (rc0) return rc0;
-  for (int i = 0; i < b->n; ++i) PIB_BHIP(b, launch_sample_fp64(sample_args(b, i, seed, nullptr), s));
+  PIB_BHIP(b, launch_sample_batch(sampler_args(b, seed, nullptr).data(), b->n, s));
   int rc = PIB_OK;
   // reference point: one launch per problem
   if (sequential_ms) {
@@ -564,13 +583,14 @@ int pib_batch_run(pib_batch* b, uint64_t seed, int64_t first_block, int nblocks,
     // launch, reduce every problem's block into sums[step][problem], advance step. Only
     // kernels are recorded (no memset or copy nodes).
     const int64_t* step = (const int64_t*)b->d_step.p;
+    const std::vector<SampleArgs> samplers = sampler_args(b, seed, step);
+    std::vector<SumArgs> sums;
+    for (int i = 0; i < b->n; ++i) sums.push_back(sum_args(b, i, step));
     PIB_BHIP(b, hipStreamBeginCapture(b->cap, hipStreamCaptureModeThreadLocal));
-    hipError_t e = hipSuccess;
-    for (int i = 0; i < b->n && e == hipSuccess; ++i) e = launch_sample_fp64(sample_args(b, i, seed, step), b->cap);
+    hipError_t e = launch_sample_batch(samplers.data(), b->n, b->cap);
     if (e == hipSuccess) e = launch_batch_eval(b, b->cap);
-    for (int i = 0; i < b->n && e == hipSuccess; ++i)
-      e = launch_block_sums(sum_args(b, i, step), (double*)b->partials.p, b->nparts,
-                            b->sums + (int64_t)i * NUM_SUMS, b->cap);
+    if (e == hipSuccess)
+      e = launch_block_sums_batch(sums.data(), b->n, (double*)b->partials.p, b->nparts, b->sums, b->cap);
     if (e == hipSuccess) {
       hipLaunchKernelGGL(k_inc_i64, dim3(1), dim3(64), 0, b->cap, (int64_t*)b->d_step.p);
       e = hipGetLastError();

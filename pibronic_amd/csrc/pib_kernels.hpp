@@ -139,6 +139,16 @@ struct SumArgs {
   int64_t max_steps;
 };
 
+// The samplers and the block sums of a batch's problems, passed by value
+constexpr int kSampleBatchProbs = 16;
+struct SampleBatch {
+  int n;
+  SampleArgs p[kSampleBatchProbs];
+};
+struct SumBatch {
+  SumArgs p[kSampleBatchProbs];
+};
+
 // Everything the lanes evaluation reads of one problem, passed by value in the kernel
 // arguments of the batched lanes kernel (at most kBatchLaunchProbs problems per launch), so
 // that every constant sits in scalar registers as in the stand-alone launch. Read from global
@@ -239,8 +249,11 @@ hipError_t launch_eval_wide_batched(int pm, const EvalArgs* probs, const BatchTi
                                     int* counter, int waves, hipStream_t s);
 constexpr int kWideMaxStates = 16;
 hipError_t launch_sample_fp64(const SampleArgs& a, hipStream_t s);
+hipError_t launch_sample_batch(const SampleArgs* args, int n, hipStream_t s);
 hipError_t launch_block_sums(const SumArgs& a, double* partials, int nparts, double* sums,
                              hipStream_t s);
+// the problems of a batch: partials holds n * nparts rows, problem i's sums go to sums + i * NUM_SUMS
+hipError_t launch_block_sums_batch(const SumArgs* args, int n, double* partials, int nparts, double* sums, hipStream_t s);
 // Partial rows of the block sums: one per work-group of k_sum_partials, at most this many
 // whatever B is (the work-groups stride over the block).
 constexpr int kSumMaxParts = 1024;

@@ -61,7 +61,7 @@ __device__ __forceinline__ void block_tree(double* sh, double (&v)[NUM_SUMS]) {
   }
 }
 
-__global__ void __launch_bounds__(kSumThreads) k_sum_partials(const SumArgs a, double* partials) {
+__device__ __forceinline__ void sum_partials(const SumArgs& a, double* partials) {
   __shared__ double sh[NUM_SUMS * kSumThreads];
   double v[NUM_SUMS];
 #pragma unroll
@@ -99,9 +99,8 @@ __global__ void __launch_bounds__(kSumThreads) k_sum_partials(const SumArgs a, d
     partials[(int64_t)blockIdx.x * NUM_SUMS + threadIdx.x] = sh[threadIdx.x * kSumThreads];
 }
 
-__global__ void __launch_bounds__(kSumThreads) k_sum_final(const double* partials, int nparts,
-                                                           double* sums, const int64_t* step,
-                                                           int64_t step_stride, int64_t max_steps) {
+__device__ __forceinline__ void sum_final(const double* partials, int nparts, double* sums, const int64_t* step,
+                                          int64_t step_stride, int64_t max_steps) {
   if (step) {
     const int64_t k = *step;
     if (k < 0 || k >= max_steps) return;  // uniform over the work-group
@@ -119,6 +118,26 @@ __global__ void __launch_bounds__(kSumThreads) k_sum_final(const double* partial
   if (threadIdx.x < NUM_SUMS) sums[threadIdx.x] = sh[threadIdx.x * kSumThreads];
 }
 
+__global__ void __launch_bounds__(kSumThreads) k_sum_partials(const SumArgs a, double* partials) {
+  sum_partials(a, partials);
+}
+__global__ void __launch_bounds__(kSumThreads) k_sum_final(const double* partials, int nparts, double* sums,
+                                                           const int64_t* step, int64_t step_stride,
+                                                           int64_t max_steps) {
+  sum_final(partials, nparts, sums, step, step_stride, max_steps);
+}
+
+// the same for the problems of a batch (grid y / x = problem): two launches for all of them
+__global__ void __launch_bounds__(kSumThreads) k_sum_partials_batched(const SumBatch b, double* partials) {
+  sum_partials(b.p[blockIdx.y], partials + (int64_t)blockIdx.y * gridDim.x * NUM_SUMS);
+}
+__global__ void __launch_bounds__(kSumThreads) k_sum_final_batched(const SumBatch b, const double* partials, int nparts,
+                                                                   double* sums) {
+  const SumArgs& a = b.p[blockIdx.x];
+  sum_final(partials + (int64_t)blockIdx.x * nparts * NUM_SUMS, nparts, sums + (int64_t)blockIdx.x * NUM_SUMS, a.step,
+            a.step_stride, a.max_steps);
+}
+
 hipError_t launch_block_sums(const SumArgs& a, double* partials, int nparts, double* sums,
                              hipStream_t s) {
   hipLaunchKernelGGL(k_sum_partials, dim3(nparts), dim3(kSumThreads), 0, s, a, partials);
@@ -127,6 +146,21 @@ hipError_t launch_block_sums(const SumArgs& a, double* partials, int nparts, dou
   hipLaunchKernelGGL(k_sum_final, dim3(1), dim3(kSumThreads), 0, s, partials, nparts, sums, a.step,
                      a.step_stride, a.max_steps);
   return hipGetLastError();
+}
+
+hipError_t launch_block_sums_batch(const SumArgs* args, int n, double* partials, int nparts, double* sums, hipStream_t s) {
+  for (int i0 = 0; i0 < n; i0 += kSampleBatchProbs) {
+    SumBatch b{};
+    const int m = n - i0 < kSampleBatchProbs ? n - i0 : kSampleBatchProbs;
+    for (int i = 0; i < m; ++i) b.p[i] = args[i0 + i];
+    double* part = partials + (int64_t)i0 * nparts * NUM_SUMS;
+    hipLaunchKernelGGL(k_sum_partials_batched, dim3(nparts, m), dim3(kSumThreads), 0, s, b, part);
+    if (hipError_t e = hipGetLastError()) return e;
+    hipLaunchKernelGGL(k_sum_final_batched, dim3(m), dim3(kSumThreads), 0, s, b, part, nparts,
+                       sums + (int64_t)i0 * NUM_SUMS);
+    if (hipError_t e = hipGetLastError()) return e;
+  }
+  return hipSuccess;
 }
 
 }  // namespace pib

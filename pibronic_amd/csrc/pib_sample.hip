@@ -23,17 +23,23 @@
 //
 // Layout: a wave takes one mode of 64 consecutive samples, one lane per row (sample, mode), so
 // the mode's factor entries are wave-uniform scalar loads. Each lane walks its beads
-// downwards in chunks of 8; a chunk is staged in LDS and the wave then writes the 64 rows'
-// chunk with consecutive lanes on consecutive addresses (64-byte row segments).
+// downwards in chunks of 8 or 16; a chunk is staged in LDS and the wave then writes the 64 rows'
+// chunk with consecutive lanes on consecutive addresses (64- or 128-byte row segments).
+#include <algorithm>
+
 #include "pib_common.hpp"
 #include "pib_kernels.hpp"
 
 namespace pib {
 
 constexpr int kSampleWaves = 4;   // waves per work-group, each independent
-constexpr int kChunk = 8;         // beads staged per lane before a coalesced write-out (64 B
-                                  // per row: LDS for ~6 waves per SIMD)
-constexpr int kLd = kChunk + 1;   // padded LDS row
+// Beads staged per lane before a write-out: 16 (a whole 128-byte line where rows start on one)
+// beyond 24 beads per row, else 8. Half lines written apart reach memory one by one once the rows
+// in flight exceed the L2; short rows lose more by the waves that the larger LDS tile displaces.
+// MI355X, us with 8 / 16, A N P samples: 4 8 64 1e5 122 / 90, 8 16 64 1e5 271 / 160, 6 12 256
+// 16,384 134 / 92, 11 17 50 32,768 74 / 61, 5 7 33 20,000 19.6 / 17.5, 2 6 24 1e5 29 / 33,
+// 3 6 16 1e5 22.0 / 22.8, 2 3 12 1e4 5.6 / 6.3.
+static bool long_rows(const SampleArgs& a) { return a.P > 24; }
 
 __device__ __forceinline__ int draw_source(const SampleArgs& a, int64_t gsample) {
   if (a.A_rho == 1) return 0;
@@ -69,88 +75,115 @@ __device__ __forceinline__ void normal_quad(uint64_t grow, int m, uint32_t k0, u
   z[3] = (double)(rb * __builtin_amdgcn_sinf(ub));
 }
 
-__global__ void __launch_bounds__(kWave * kSampleWaves) k_sample_fp64(const SampleArgs a) {
-  __shared__ double stage_all[kSampleWaves][kWave * kLd];
+// one unit of work of a wave: mode u % N of the sample group u / N
+template <int CHUNK>
+__device__ __forceinline__ void sample_unit(const SampleArgs& a, int64_t u, int64_t offset, int lane, double* stage) {
   const int P = a.P, N = a.N;
-  const int64_t groups = (a.B + kWave - 1) / kWave;  // groups of 64 consecutive samples
-  const int64_t units = groups * N;                  // (sample group, mode) pairs
+  constexpr int ld = CHUNK + 1;  // padded LDS row
+  // wave-uniform: the sample group and the mode; every lane of the wave runs the same chunks
+  const int64_t sg = u / N;
+  const int j = (int)(u - sg * N);
+  const int64_t s0 = sg * kWave;
+  const int64_t s = s0 + lane;
+  const bool live = s < a.B;
+  const int64_t gs = offset + (live ? s : s0);
+  const int src = live ? draw_source(a, gs) : 0;
+  const uint64_t grow = (uint64_t)gs * (uint64_t)N + (uint64_t)j;
+  // the mode's factor entries are the same for the whole wave: read through the constant
+  // address space (the kernel never writes them), so they come by scalar loads
+  typedef const double __attribute__((address_space(4))) cdouble;
+  cdouble* dinv = (cdouble*)(a.chol + (int64_t)j * 3 * P);
+  cdouble* sub = dinv + P;
+  cdouble* last = sub + P;
+  const double d = a.shift[src * N + j];
+  if (live && a.src && j == 0) a.src[s] = src;
+  const int nrow = (a.B - s0) < kWave ? (int)(a.B - s0) : kWave;
+  const int64_t rstride = (int64_t)N * P;
+  double zq[4], xl = 0.0, xn = 0.0;
+  // beads in descending order, in chunks [kb, ke) aligned to multiples of CHUNK, and within
+  // a chunk quad by quad. One formula for every bead: the host stores sub[k] = 0 for
+  // k >= P-2 and last[P-1] = 0, and x_{P-1} (xl) and x_{k+1} (xn) start at 0, so bead P-1
+  // gives z dinv and bead P-2 (z - last xl) dinv exactly.
+  // Lanes past the block's end (the last group only) run the same uniform loop on the
+  // group's first sample; their rows are never written out.
+  for (int kb = ((P - 1) / CHUNK) * CHUNK; kb >= 0; kb -= CHUNK) {
+    const int ke = kb + CHUNK < P ? kb + CHUNK : P;
+#pragma unroll 2
+    for (int m = (ke - 1) >> 2; m >= (kb >> 2); --m) {
+      double cd[4], cs[4], cl[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int k = 4 * m + e < P ? 4 * m + e : P - 1;  // the top quad may be partial
+        cd[e] = dinv[k];
+        cs[e] = sub[k];
+        cl[e] = last[k];
+      }
+      normal_quad(grow, m, a.key0, a.key1, zq);
+#pragma unroll
+      for (int e = 3; e >= 0; --e) {
+        const int k = 4 * m + e;
+        if (k < ke) {  // uniform over the wave
+          const double x = fma(-cl[e], xl, fma(-cs[e], xn, zq[e])) * cd[e];
+          if (k == P - 1) xl = x;
+          xn = x;
+          stage[lane * ld + (k - kb)] = x + d;
+        }
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    // write out: row rr (sample s0 + rr, mode j) has its beads contiguous in q
+    const int w_ = ke - kb;
+    double* __restrict__ qj = a.q + (s0 * N + j) * (int64_t)P + kb;
+    if (w_ == CHUNK && nrow == kWave) {  // full chunk: no divisions
+#pragma unroll 4
+      for (int it = 0; it < CHUNK; ++it) {
+        const int e = lane + kWave * it, rr = e / CHUNK, kk = e % CHUNK;
+        qj[rr * rstride + kk] = stage[rr * ld + kk];
+      }
+    } else {
+      for (int e = lane; e < nrow * w_; e += kWave) {
+        const int rr = e / w_, kk = e - rr * w_;
+        qj[rr * rstride + kk] = stage[rr * ld + kk];
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  }
+}
+
+template <int CHUNK>
+__global__ void __launch_bounds__(kWave * kSampleWaves) k_sample_fp64(const SampleArgs a) {
+  __shared__ double stage_all[kSampleWaves][kWave * (CHUNK + 1)];
+  const int64_t units = (a.B + kWave - 1) / kWave * a.N;  // (sample group, mode) pairs
   const int lane = threadIdx.x & (kWave - 1);
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);  // wave-uniform
-  double* stage = stage_all[w];
   const int64_t offset = a.step ? a.offset + *a.step * a.B : a.offset;
-  for (int64_t u = (int64_t)blockIdx.x * kSampleWaves + w; u < units; u += (int64_t)gridDim.x * kSampleWaves) {
-    // wave-uniform: the sample group and the mode; every lane of the wave runs the same chunks
-    const int64_t sg = u / N;
-    const int j = (int)(u - sg * N);
-    const int64_t s0 = sg * kWave;
-    const int64_t s = s0 + lane;
-    const bool live = s < a.B;
-    const int64_t gs = offset + (live ? s : s0);
-    const int src = live ? draw_source(a, gs) : 0;
-    const uint64_t grow = (uint64_t)gs * (uint64_t)N + (uint64_t)j;
-    // the mode's factor entries are the same for the whole wave: read through the constant
-    // address space (the kernel never writes them), so they come by scalar loads
-    typedef const double __attribute__((address_space(4))) cdouble;
-    cdouble* dinv = (cdouble*)(a.chol + (int64_t)j * 3 * P);
-    cdouble* sub = dinv + P;
-    cdouble* last = sub + P;
-    const double d = a.shift[src * N + j];
-    if (live && a.src && j == 0) a.src[s] = src;
-    const int nrow = (a.B - s0) < kWave ? (int)(a.B - s0) : kWave;
-    double zq[4], xl = 0.0, xn = 0.0;
-    // beads in descending order, in chunks [kb, ke) aligned to multiples of kChunk, and within
-    // a chunk quad by quad. One formula for every bead: the host stores sub[k] = 0 for
-    // k >= P-2 and last[P-1] = 0, and x_{P-1} (xl) and x_{k+1} (xn) start at 0, so bead P-1
-    // gives z dinv and bead P-2 (z - last xl) dinv exactly.
-    // Lanes past the block's end (the last group only) run the same uniform loop on the
-    // group's first sample; their rows are never written out.
-    for (int kb = ((P - 1) / kChunk) * kChunk; kb >= 0; kb -= kChunk) {
-      const int ke = kb + kChunk < P ? kb + kChunk : P;
-#pragma unroll 2
-      for (int m = (ke - 1) >> 2; m >= (kb >> 2); --m) {
-        double cd[4], cs[4], cl[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int k = 4 * m + e < P ? 4 * m + e : P - 1;  // the top quad may be partial
-          cd[e] = dinv[k];
-          cs[e] = sub[k];
-          cl[e] = last[k];
-        }
-        normal_quad(grow, m, a.key0, a.key1, zq);
-#pragma unroll
-        for (int e = 3; e >= 0; --e) {
-          const int k = 4 * m + e;
-          if (k < ke) {  // uniform over the wave
-            const double x = fma(-cl[e], xl, fma(-cs[e], xn, zq[e])) * cd[e];
-            if (k == P - 1) xl = x;
-            xn = x;
-            stage[lane * kLd + (k - kb)] = x + d;
-          }
-        }
-      }
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      // write the chunk: row rr (sample s0 + rr, mode j) has its beads [kb, ke) contiguous in q
-      const int w_ = ke - kb;
-      double* __restrict__ qj = a.q + (s0 * N + j) * (int64_t)P + kb;
-      const int64_t rstride = (int64_t)N * P;
-      if (w_ == kChunk && nrow == kWave) {  // full chunk: no divisions
-#pragma unroll 4
-        for (int it = 0; it < kChunk; ++it) {
-          const int e = lane + kWave * it, rr = e / kChunk, kk = e % kChunk;
-          qj[rr * rstride + kk] = stage[rr * kLd + kk];
-        }
-      } else {
-        for (int e = lane; e < nrow * w_; e += kWave) {
-          const int rr = e / w_, kk = e - rr * w_;
-          qj[rr * rstride + kk] = stage[rr * kLd + kk];
-        }
-      }
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  for (int64_t u = (int64_t)blockIdx.x * kSampleWaves + w; u < units; u += (int64_t)gridDim.x * kSampleWaves)
+    sample_unit<CHUNK>(a, u, offset, lane, stage_all[w]);
+}
+
+// The samplers of several problems (the temperatures of a batch) in one launch: one problem's
+// rows alone leave the chip mostly waiting on each wave's serial walk over the beads. Sixteen
+// temperatures of A = 6, N = 12, P = 52..256, 16,384 samples each (MI355X): 1.69 ms as sixteen
+// launches with half-line write-out, 1.53 as one with whole lines (3.9 GB written; a fill reaches 6.7 TB/s).
+// The caller puts the longest rows first, so that the short ones fill the tail.
+template <int CHUNK>
+__global__ void __launch_bounds__(kWave * kSampleWaves) k_sample_batched(const SampleBatch b) {
+  __shared__ double stage_all[kSampleWaves][kWave * (CHUNK + 1)];
+  const int lane = threadIdx.x & (kWave - 1);
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  int64_t u = (int64_t)blockIdx.x * kSampleWaves + w;
+  for (int i = 0; i < b.n; ++i) {  // wave-uniform
+    const SampleArgs& a = b.p[i];
+    const int64_t units = (a.B + kWave - 1) / kWave * a.N;
+    if (u < units) {
+      sample_unit<CHUNK>(a, u, a.step ? a.offset + *a.step * a.B : a.offset, lane, stage_all[w]);
+      return;
     }
+    u -= units;
   }
 }
 
@@ -159,8 +192,37 @@ hipError_t launch_sample_fp64(const SampleArgs& a, hipStream_t s) {
   int64_t groups = (units + kSampleWaves - 1) / kSampleWaves;
   if (groups > 65536) groups = 65536;
   if (groups < 1) groups = 1;
-  hipLaunchKernelGGL(k_sample_fp64, dim3((unsigned)groups), dim3(kWave * kSampleWaves), 0, s, a);
+  if (long_rows(a))
+    hipLaunchKernelGGL(k_sample_fp64<16>, dim3((unsigned)groups), dim3(kWave * kSampleWaves), 0, s, a);
+  else
+    hipLaunchKernelGGL(k_sample_fp64<8>, dim3((unsigned)groups), dim3(kWave * kSampleWaves), 0, s, a);
   return hipGetLastError();
+}
+
+hipError_t launch_sample_batch(const SampleArgs* args, int n, hipStream_t s) {
+  for (int i0 = 0; i0 < n; i0 += kSampleBatchProbs) {
+    SampleBatch b{};
+    b.n = std::min(kSampleBatchProbs, n - i0);
+    int64_t units = 0;
+    bool lng = false;
+    for (int i = 0; i < b.n; ++i) {
+      b.p[i] = args[i0 + i];
+      lng = lng || long_rows(b.p[i]);
+      units += (b.p[i].B + kWave - 1) / kWave * b.p[i].N;
+    }
+    const int64_t groups = (units + kSampleWaves - 1) / kSampleWaves;
+    if (groups > 65536 * kSampleBatchProbs) {  // beyond one launch's grid: the strided launches
+      for (int i = 0; i < b.n; ++i)
+        if (hipError_t e = launch_sample_fp64(b.p[i], s)) return e;
+      continue;
+    }
+    if (lng)
+      hipLaunchKernelGGL(k_sample_batched<16>, dim3((unsigned)groups), dim3(kWave * kSampleWaves), 0, s, b);
+    else
+      hipLaunchKernelGGL(k_sample_batched<8>, dim3((unsigned)groups), dim3(kWave * kSampleWaves), 0, s, b);
+    if (hipError_t e = hipGetLastError()) return e;
+  }
+  return hipSuccess;
 }
 
 }  // namespace pib
