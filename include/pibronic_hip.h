@@ -298,6 +298,29 @@ int pib_flow_layer_fused_frag(pib_ctx* ctx, int inverse, int64_t B, int D, int h
                               const uint16_t* W3_frag_dev, const float* b1_dev, const float* b2_dev,
                               const float* b3_dev, void* stream);
 
+/* Training pass of the whole flow with BF16x3 products, where pib_flow_train_supported is 1 (L >= 2
+ * layers, D a multiple of 128, hidden and B of 64, 64 (D + 2 hidden + 24) bytes within 160 KB, not
+ * both a small net and more than 4,096 samples) and all float buffers are 16-byte aligned;
+ * PIB_ERR_UNSUPPORTED otherwise. params: per layer W1 (D/2 x hidden), b1, W2 (hidden x hidden), b2,
+ * W3 (hidden x D), b3; even layers transform the upper half. Forward: the inverse flow of z0 (B*D,
+ * whitened samples) into z1 and logdet (double, B; the inverse map's), keeping halves
+ * (L-2, B, D/2), h1 and h2 (L, B, hidden), o (L, B, D) and frags (the weights in product order,
+ * 4 L (D/2 hidden + hidden^2 + hidden D) uint16) for the backward. */
+int pib_flow_train_supported(pib_ctx* ctx, int64_t B, int D, int hidden, int L);
+int pib_flow_train_forward(pib_ctx* ctx, int64_t B, int D, int hidden, int L, float smax,
+                           const float* params_dev, float* z0_dev, float* z1_dev, float* halves_dev,
+                           float* h1_dev, float* h2_dev, float* o_dev, uint16_t* frags_dev,
+                           double* logdet_dev, void* stream);
+
+/* Backward of L = -sum_b c_b (log rho(R0_b) + logdet_b): dz (B*D) holds the gradient at z1 (from
+ * log rho) and is overwritten, as is o; dh1 and dh2 (L, B, hidden) are scratch; grad (as params)
+ * is written whole. */
+int pib_flow_train_backward(pib_ctx* ctx, int64_t B, int D, int hidden, int L, float smax,
+                            const float* params_dev, float* grad_dev, float* z0_dev, float* z1_dev,
+                            float* halves_dev, float* h1_dev, float* h2_dev, float* o_dev,
+                            float* dz_dev, float* dh1_dev, float* dh2_dev, uint16_t* frags_dev,
+                            const double* c_dev, void* stream);
+
 /* Base distribution of the flow drawn directly in its whitened, permuted coordinates: the
  * harmonic rho is the mixture sum_a w_a N(mu_a, I) there (mu_a (D, double) = the surface's
  * displacement d_a - m rotated by the circulant basis and divided by sigma; w_a the sampler's

@@ -68,6 +68,9 @@ SIGNATURES = {
                                    _vp, _vp, _vp, _vp]),
     "pib_flow_coupling_inverse_backward": (_c_int, [_vp, _c_i64, _c_int, _c_int, _c_int,
                                                     ctypes.c_float, _vp, _vp, _vp, _vp, _vp, _vp]),
+    "pib_flow_train_supported": (_c_int, [_vp, _c_i64, _c_int, _c_int, _c_int]),
+    "pib_flow_train_forward": (_c_int, [_vp, _c_i64, _c_int, _c_int, _c_int, ctypes.c_float] + [_vp] * 10),
+    "pib_flow_train_backward": (_c_int, [_vp, _c_i64, _c_int, _c_int, _c_int, ctypes.c_float] + [_vp] * 14),
     "pib_flow_logrho": (_c_int, [_vp, _c_i64, _vp, _vp, _vp, _vp, _vp]),
     "pib_colsum_f32": (_c_int, [_vp, _c_i64, _c_i64, _vp, _c_i64, _vp, _vp]),
     "pib_adam_f32": (_c_int, [_vp, _c_i64, _vp, _vp, _vp, _vp, ctypes.c_float, ctypes.c_float,
@@ -307,6 +310,20 @@ class Context:
         self._check(self.lib.pib_flow_coupling_inverse_backward(
             self.h, int(B), int(D), int(a_off), int(b_off), float(smax), _devptr(y), _devptr(o),
             _devptr(dz), _devptr(dout), _devptr(c), _stream(stream)))
+
+    def flow_train_supported(self, B, D, hidden, L):
+        return bool(self.lib.pib_flow_train_supported(self.h, int(B), int(D), int(hidden), int(L)))
+
+    def flow_train_forward(self, B, D, hidden, L, smax, params, z0, z1, halves, h1, h2, o, frags, logdet, stream=None):
+        self._check(self.lib.pib_flow_train_forward(
+            self.h, int(B), int(D), int(hidden), int(L), float(smax),
+            *(_devptr(x) for x in (params, z0, z1, halves, h1, h2, o, frags, logdet)), _stream(stream)))
+
+    def flow_train_backward(self, B, D, hidden, L, smax, params, grad, z0, z1, halves, h1, h2, o, dz, dh1, dh2, frags, c,
+                            stream=None):
+        self._check(self.lib.pib_flow_train_backward(
+            self.h, int(B), int(D), int(hidden), int(L), float(smax),
+            *(_devptr(x) for x in (params, grad, z0, z1, halves, h1, h2, o, dz, dh1, dh2, frags, c)), _stream(stream)))
 
     def flow_set_base(self, mu, c):
         """mu (A_rho, D) and c (A_rho,) of the flow's base distribution (float64 host arrays)."""

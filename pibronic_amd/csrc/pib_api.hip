@@ -955,6 +955,56 @@ int pib_flow_coupling_inverse_backward(pib_ctx* c, int64_t B, int D, int a_off, 
   return PIB_OK;
 }
 
+static int train_check(pib_ctx* c, const TrainArgs& a, const char* who) {
+  if (!(a.smax > 0.0f) || !train_supported(a, c->num_cu))
+    return fail(c, PIB_ERR_UNSUPPORTED, std::string(who) + ": needs L >= 2, D a multiple of 128, hidden and B of 64, "
+                                                           "smax > 0, 16-byte aligned buffers, 16 rows of the products "
+                                                           "in LDS and enough weights for the samples");
+  return PIB_OK;
+}
+
+int pib_flow_train_supported(pib_ctx* c, int64_t B, int D, int hidden, int L) {
+  if (!c) return 0;
+  TrainArgs a{};
+  a.B = B; a.D = D; a.hidden = hidden; a.L = L;
+  return train_supported(a, c->num_cu) ? 1 : 0;
+}
+
+int pib_flow_train_forward(pib_ctx* c, int64_t B, int D, int hidden, int L, float smax, const float* params,
+                           float* z0, float* z1, float* halves, float* h1, float* h2, float* o, uint16_t* frags,
+                           double* logdet, void* stream) {
+  if (!c) return PIB_ERR_ARG;
+  if (!params || !z0 || !z1 || (L > 2 && !halves) || !h1 || !h2 || !o || !frags || !logdet)
+    return fail(c, PIB_ERR_ARG, "flow_train_forward: null pointer");
+  TrainArgs a{};
+  a.B = B; a.D = D; a.hidden = hidden; a.L = L; a.smax = smax; a.params = params;
+  a.z0 = z0; a.z1 = z1; a.halves = halves; a.h1 = h1; a.h2 = h2; a.o = o; a.logdet = logdet;
+  a.fwd = frags; a.bwd = frags + train_frags(a) / 4;
+  if (int r = train_check(c, a, "flow_train_forward")) return r;
+  PIB_HIP(c, hipSetDevice(c->device));
+  hipError_t e = launch_train_forward(a, c->num_cu, (hipStream_t)stream);
+  if (e != hipSuccess) return hip_fail(c, e, "flow_train_forward launch");
+  return PIB_OK;
+}
+
+int pib_flow_train_backward(pib_ctx* c, int64_t B, int D, int hidden, int L, float smax, const float* params,
+                            float* grad, float* z0, float* z1, float* halves, float* h1, float* h2, float* o,
+                            float* dz, float* dh1, float* dh2, uint16_t* frags, const double* cb, void* stream) {
+  if (!c) return PIB_ERR_ARG;
+  if (!params || !grad || !z0 || !z1 || (L > 2 && !halves) || !h1 || !h2 || !o || !dz || !dh1 || !dh2 || !frags || !cb)
+    return fail(c, PIB_ERR_ARG, "flow_train_backward: null pointer");
+  TrainArgs a{};
+  a.B = B; a.D = D; a.hidden = hidden; a.L = L; a.smax = smax; a.params = params; a.grad = grad;
+  a.z0 = z0; a.z1 = z1; a.halves = halves; a.h1 = h1; a.h2 = h2; a.o = o; a.dz = dz; a.dh1 = dh1; a.dh2 = dh2;
+  a.c = cb;
+  a.fwd = frags; a.bwd = frags + train_frags(a) / 4;
+  if (int r = train_check(c, a, "flow_train_backward")) return r;
+  PIB_HIP(c, hipSetDevice(c->device));
+  hipError_t e = launch_train_backward(a, c->num_cu, (hipStream_t)stream);
+  if (e != hipSuccess) return hip_fail(c, e, "flow_train_backward launch");
+  return PIB_OK;
+}
+
 int pib_flow_set_base(pib_ctx* c, int A_rho, int D, const double* mu, const double* cc) {
   if (!c) return PIB_ERR_ARG;
   if (A_rho < 1 || A_rho > 16 || D < 2 || (D & 1) || !mu || !cc)

@@ -143,6 +143,29 @@ struct LogRhoArgs {
   double* logrho;         // (B,) or nullptr
 };
 
+// Training pass of the whole flow (pib_train.hip); buffers as in pib_flow_train_forward
+struct TrainArgs {
+  int64_t B;
+  int D, hidden, L;
+  float smax;
+  const float* params;
+  float* grad;
+  float* z0;       // (B, D) whitened samples
+  float* z1;       // (B, D) the inverse flow's result
+  float* halves;   // (L - 2, B, D / 2)
+  float *h1, *h2;  // (L, B, hidden)
+  float* o;        // (L, B, D); after the backward the gradients there
+  float* dz;       // (B, D) in: gradient at z1
+  float *dh1, *dh2;
+  double* logdet;  // (B,)
+  const double* c;
+  unsigned short *fwd, *bwd;  // the weights in product order, train_frags bytes together
+};
+bool train_supported(const TrainArgs& a, int num_cu);
+size_t train_frags(const TrainArgs& a);
+hipError_t launch_train_forward(const TrainArgs& a, int num_cu, hipStream_t s);
+hipError_t launch_train_backward(const TrainArgs& a, int num_cu, hipStream_t s);
+
 hipError_t launch_logrho(const LogRhoArgs& a, hipStream_t s);
 hipError_t launch_adam_f32(int64_t n, float* p, const float* g, float* m, float* v, float lr,
                            float b1, float b2, float eps, int step, hipStream_t s);

@@ -12,6 +12,7 @@
 // Shapes must be multiples of the tile (M, N of 64, K of 16); the launcher checks.
 #include "pib_common.hpp"
 #include "pib_flow.hpp"
+#include "pib_gemm3.hpp"
 
 #include <algorithm>
 
@@ -242,135 +243,34 @@ __global__ void __launch_bounds__(256) k_gemm_bf16x3(GemmArgs g) {
     }
 }
 
-// Pipelined BF16x3 variant for 16-byte aligned operands: float4 global loads, and the next K
-// slab is loaded into registers while the matrix cores work on the current one.
+// 16-byte aligned operands: the pipelined tiles of pib_gemm3.hpp. MI355X, us with slabs of 32 in one
+// buffer and 2- and 8-byte LDS writes / these: 2,048 x 1,024 x 256 16.0 / 11.8, 32,768 x 256 x 512 84.7 / 61.2,
+// 2,048 x 256 x 1,024 (B transposed) 19.0 / 15.1, 512 x 256 x 32,768 (A transposed) 172 / 78.
 template <bool TA, bool TB>
 __global__ void __launch_bounds__(256) k_gemm_bf16x3_v(GemmArgs g) {
-  __shared__ __align__(16) unsigned short Ah[kTM][kLd3], Al[kTM][kLd3];
-  __shared__ __align__(16) unsigned short Bh[kTN][kLd3], Bl[kTN][kLd3];
-  const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6;
-  const int wr = wave >> 1, wc = wave & 1;
+  extern __shared__ __align__(16) unsigned char lds3[];
+  const int t = threadIdx.x, lane = t & 63, wr = t >> 7, wc = (t >> 6) & 1;
   const int64_t m0 = (int64_t)blockIdx.y * kTM, n0 = (int64_t)blockIdx.x * kTN;
   const int64_t kbeg = g.partial ? (int64_t)blockIdx.z * g.kchunk : 0;
   const int64_t kend = g.partial ? kbeg + g.kchunk : g.K;
-  f32x4 acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  // slab element groups (4 floats each) of this thread: q = tid + 256 r, r = 0, 1
-  float4 ra[2], rb[2];
-  auto load = [&](int64_t k0) {
-#pragma unroll
-    for (int r = 0; r < 2; ++r) {
-      const int q = tid + 256 * r;
-      if (TA) {  // A stored K x M: 4 consecutive m
-        const int k = q / 16, i = (q % 16) * 4;
-        ra[r] = *(const float4*)(g.A + (k0 + k) * g.lda + m0 + i);
-      } else {   // A stored M x K: 4 consecutive k
-        const int i = q / 8, k = (q % 8) * 4;
-        ra[r] = *(const float4*)(g.A + (m0 + i) * g.lda + k0 + k);
-      }
-      if (TB) {  // B stored N x K: 4 consecutive k
-        const int j = q / 8, k = (q % 8) * 4;
-        rb[r] = *(const float4*)(g.B + (n0 + j) * g.ldb + k0 + k);
-      } else {   // B stored K x N: 4 consecutive n
-        const int k = q / 16, j = (q % 16) * 4;
-        rb[r] = *(const float4*)(g.B + (k0 + k) * g.ldb + n0 + j);
-      }
-    }
-  };
-  auto split = [](float x, unsigned short& h, unsigned short& l) {
-    h = f2bf(x);
-    l = f2bf(x - bf2f(h));
-  };
-  auto store = [&]() {
-#pragma unroll
-    for (int r = 0; r < 2; ++r) {
-      const int q = tid + 256 * r;
-      const float av[4] = {ra[r].x, ra[r].y, ra[r].z, ra[r].w};
-      const float bv[4] = {rb[r].x, rb[r].y, rb[r].z, rb[r].w};
-      unsigned short h[4], l[4];
-      if (TA) {
-        const int k = q / 16, i = (q % 16) * 4;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) { split(av[e], h[e], l[e]); Ah[i + e][k] = h[e]; Al[i + e][k] = l[e]; }
-      } else {
-        const int i = q / 8, k = (q % 8) * 4;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) split(av[e], h[e], l[e]);
-        *(uint2*)&Ah[i][k] = make_uint2(h[0] | ((unsigned)h[1] << 16), h[2] | ((unsigned)h[3] << 16));
-        *(uint2*)&Al[i][k] = make_uint2(l[0] | ((unsigned)l[1] << 16), l[2] | ((unsigned)l[3] << 16));
-      }
-      if (TB) {
-        const int j = q / 8, k = (q % 8) * 4;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) split(bv[e], h[e], l[e]);
-        *(uint2*)&Bh[j][k] = make_uint2(h[0] | ((unsigned)h[1] << 16), h[2] | ((unsigned)h[3] << 16));
-        *(uint2*)&Bl[j][k] = make_uint2(l[0] | ((unsigned)l[1] << 16), l[2] | ((unsigned)l[3] << 16));
-      } else {
-        const int k = q / 16, j = (q % 16) * 4;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) { split(bv[e], h[e], l[e]); Bh[j + e][k] = h[e]; Bl[j + e][k] = l[e]; }
-      }
-    }
-  };
-
-  load(kbeg);
-  for (int64_t k0 = kbeg; k0 < kend; k0 += kTK3) {
-    store();
-    __syncthreads();
-    if (k0 + kTK3 < kend) load(k0 + kTK3);  // in flight during the matrix-core work below
-    const int kq = 8 * (lane >> 4);
-    bf16x8 ah[2], al[2], bh[2], bl[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int r = wr * 32 + i * 16 + (lane & 15);
-      ah[i] = __builtin_bit_cast(bf16x8, *(const uvec4*)&Ah[r][kq]);
-      al[i] = __builtin_bit_cast(bf16x8, *(const uvec4*)&Al[r][kq]);
-    }
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int c = wc * 32 + j * 16 + (lane & 15);
-      bh[j] = __builtin_bit_cast(bf16x8, *(const uvec4*)&Bh[c][kq]);
-      bl[j] = __builtin_bit_cast(bf16x8, *(const uvec4*)&Bl[c][kq]);
-    }
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[i], bh[j], acc[i][j], 0, 0, 0);
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[i], bl[j], acc[i][j], 0, 0, 0);
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[i], bh[j], acc[i][j], 0, 0, 0);
-      }
-    __syncthreads();
-  }
-  if (g.partial) {
-    float* P = g.partial + (int64_t)blockIdx.z * g.M * g.N;
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const int64_t col = n0 + wc * 32 + j * 16 + (lane & 15);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int64_t row = m0 + wr * 32 + i * 16 + 4 * (lane >> 4) + r;
-          P[row * g.N + col] = acc[i][j][r];
-        }
-      }
-    return;
-  }
+  const float* pa = TA ? g.A + m0 + (t & 63) : g.A + (m0 + (t >> 3)) * g.lda;
+  const float* pb = TB ? g.B + (n0 + (t >> 3)) * g.ldb : g.B + n0 + (t & 63);
+  f32x4t acc[2][2];
+  tile3<TA, !TB>(pa, g.lda, pb, g.ldb, kbeg, kend, t, (Stage3*)lds3, acc);
+  float* P = g.partial ? g.partial + (int64_t)blockIdx.z * g.M * g.N : nullptr;
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       const int64_t col = n0 + wc * 32 + j * 16 + (lane & 15);
-      const float bv = g.bias ? g.bias[col] : 0.f;
+      const float bv = !P && g.bias ? g.bias[col] : 0.f;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int64_t row = m0 + wr * 32 + i * 16 + 4 * (lane >> 4) + r;
+        if (P) {
+          P[row * g.N + col] = acc[i][j][r];
+          continue;
+        }
         float v = acc[i][j][r] + bv;
         if (g.relu) v = v > 0.f ? v : 0.f;
         if (g.mask) v = g.mask[row * g.ldmask + col] > 0.f ? v : 0.f;
@@ -378,6 +278,14 @@ __global__ void __launch_bounds__(256) k_gemm_bf16x3_v(GemmArgs g) {
         g.C[row * g.ldc + col] = v;
       }
     }
+}
+
+template <bool TA, bool TB>
+static hipError_t launch_x3_v(const GemmArgs& g, dim3 grid, hipStream_t s) {
+  static unsigned long long lds_set = 0;
+  if (hipError_t e = ensure_dynamic_lds((const void*)k_gemm_bf16x3_v<TA, TB>, kTile3Lds, lds_set)) return e;
+  hipLaunchKernelGGL((k_gemm_bf16x3_v<TA, TB>), grid, dim3(256), kTile3Lds, s, g);
+  return hipGetLastError();
 }
 
 static bool aligned16(const void* p, int64_t ld) {
@@ -395,11 +303,12 @@ hipError_t launch_gemm_f32(bool ta, bool tb, const GemmArgs& g, hipStream_t s) {
   const int64_t kq = g.bf16x3 ? kTK3 : kTK;
   if (g.partial && (g.kchunk <= 0 || g.kchunk % kq || g.K % g.kchunk)) return hipErrorInvalidValue;
   const dim3 grid((unsigned)(g.N / kTN), (unsigned)(g.M / kTM), (unsigned)splits);
+  hipError_t ve = hipSuccess;
   if (g.bf16x3 && aligned16(g.A, g.lda) && aligned16(g.B, g.ldb)) {
-    if (!ta && !tb) hipLaunchKernelGGL((k_gemm_bf16x3_v<false, false>), grid, dim3(256), 0, s, g);
-    else if (!ta && tb) hipLaunchKernelGGL((k_gemm_bf16x3_v<false, true>), grid, dim3(256), 0, s, g);
-    else if (ta && !tb) hipLaunchKernelGGL((k_gemm_bf16x3_v<true, false>), grid, dim3(256), 0, s, g);
-    else hipLaunchKernelGGL((k_gemm_bf16x3_v<true, true>), grid, dim3(256), 0, s, g);
+    if (!ta && !tb) ve = launch_x3_v<false, false>(g, grid, s);
+    else if (!ta && tb) ve = launch_x3_v<false, true>(g, grid, s);
+    else if (ta && !tb) ve = launch_x3_v<true, false>(g, grid, s);
+    else ve = launch_x3_v<true, true>(g, grid, s);
   } else if (g.bf16x3) {
     if (!ta && !tb) hipLaunchKernelGGL((k_gemm_bf16x3<false, false>), grid, dim3(256), 0, s, g);
     else if (!ta && tb) hipLaunchKernelGGL((k_gemm_bf16x3<false, true>), grid, dim3(256), 0, s, g);
@@ -409,7 +318,7 @@ hipError_t launch_gemm_f32(bool ta, bool tb, const GemmArgs& g, hipStream_t s) {
   else if (!ta && tb) hipLaunchKernelGGL((k_gemm_f32<false, true>), grid, dim3(256), 0, s, g);
   else if (ta && !tb) hipLaunchKernelGGL((k_gemm_f32<true, false>), grid, dim3(256), 0, s, g);
   else hipLaunchKernelGGL((k_gemm_f32<true, true>), grid, dim3(256), 0, s, g);
-  hipError_t e = hipGetLastError();
+  hipError_t e = ve != hipSuccess ? ve : hipGetLastError();
   if (e != hipSuccess || !g.partial) return e;
   const int64_t MN = g.M * g.N;
   const unsigned blocks = (unsigned)std::min<int64_t>((MN + 255) / 256, 4096);

@@ -333,6 +333,11 @@ class Flow:
         self.ctx.flow_logrho(B, R0, logrho=logrho, stream=stream)
         return logrho + logdet, R0
 
+    def _train_ok(self, B):
+        """Whether the training pass of pib_flow_train_forward / _backward takes this batch."""
+        return (self.gemm == "bf16x3" and self.ctx.flow_train_supported(B, self.D, self.hidden, self.layers)
+                and self.params.data_ptr() % 16 == 0 and self.grad.data_ptr() % 16 == 0)
+
     def loss_and_grad(self, R, c, stream=None):
         """Loss -sum_b c_b log q(R_b) and its gradient (into self.grad) for fixed R, c."""
         import torch
@@ -341,25 +346,37 @@ class Flow:
         D, H, h, L = self.D, self.H, self.hidden, self.layers
         ctx = self.ctx
         c = c.to(dtype=torch.float64)
-        ys = self._buf("ys", (L, B, D))
         h1s, h2s, os_ = self._buf("h1s", (L, B, h)), self._buf("h2s", (L, B, h)), self._buf("os", (L, B, D))
-        zp = self._buf("zp", (B, D))
+        zp, dz = self._buf("zp", (B, D)), self._buf("dz", (B, D))
         work = self._buf("work", (2 * B * D,))
-        logdet = torch.zeros(B, dtype=torch.float64, device=self.dev)
         R0 = self._buf("R0", (B, self.N, self.P), torch.float64)
         ctx.flow_whiten(_native.FLOW_WHITEN, B, R, work, zp, stream)
-        for l in reversed(range(L)):
-            a_off, b_off = self.halves(l)
-            ys[l].copy_(zp)
-            self._mlp(l, zp, B, h1s[l], h2s[l], os_[l], stream)
-            ctx.flow_coupling(True, B, D, a_off, b_off, self.smax, zp, os_[l], logdet, stream)
-        ctx.flow_whiten(_native.FLOW_UNWHITEN, B, zp, work, R0, stream)
+        native = self._train_ok(B)
+        if native:
+            logdet = torch.empty(B, dtype=torch.float64, device=self.dev)
+            z1, halves = self._buf("z1", (B, D)), self._buf("halves", (max(1, L - 2), B, H))
+            frags = self._buf("frags", (4 * L * (H * h + h * h + h * D),), torch.int16)
+            ctx.flow_train_forward(B, D, h, L, self.smax, self.params, zp, z1, halves, h1s, h2s, os_, frags, logdet,
+                                   stream)
+        else:
+            logdet = torch.zeros(B, dtype=torch.float64, device=self.dev)
+            ys, z1 = self._buf("ys", (L, B, D)), zp
+            for l in reversed(range(L)):
+                a_off, b_off = self.halves(l)
+                ys[l].copy_(zp)
+                self._mlp(l, zp, B, h1s[l], h2s[l], os_[l], stream)
+                ctx.flow_coupling(True, B, D, a_off, b_off, self.smax, zp, os_[l], logdet, stream)
+        ctx.flow_whiten(_native.FLOW_UNWHITEN, B, z1, work, R0, stream)
         logrho = torch.empty(B, dtype=torch.float64, device=self.dev)
         dR0 = self._buf("dR0", (B, self.N, self.P))
         ctx.flow_logrho(B, R0, c=c, dR=dR0, logrho=logrho, stream=stream)
         loss = -(c * (logrho + logdet)).sum()
-        dz = self._buf("dz", (B, D))
         ctx.flow_whiten(_native.FLOW_GRAD, B, dR0, work, dz, stream)
+        if native:
+            dh1s, dh2s = self._buf("dh1s", (L, B, h)), self._buf("dh2s", (L, B, h))
+            ctx.flow_train_backward(B, D, h, L, self.smax, self.params, self.grad, zp, z1, halves, h1s, h2s, os_, dz,
+                                    dh1s, dh2s, frags, c, stream)
+            return loss
         dout = self._buf("dout", (B, D))
         dh2, dh1 = self._buf("dh2", (B, h)), self._buf("dh1", (B, h))
         g = self.grad
