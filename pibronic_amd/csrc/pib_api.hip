@@ -186,6 +186,8 @@ hipError_t launch_eval(const pib_ctx* c, int flags, bool wide, const EvalArgs& a
   const int pm = (flags & PIB_EVAL_PM) ? 1 : 0;
   if (flags & PIB_EVAL_FP32) return launch_eval_fp32(a.A, a.AR, pm, a, s);
   if (uses_block(c, flags)) return launch_eval_block(pm, block_args(c, a, pm != 0), s);
+  if (wide && !pm && !(flags & (PIB_EVAL_WIDE | PIB_EVAL_BF16X3)) && wide4_supported(a, c->num_cu))
+    return launch_eval_wide4(a, s);
   if (wide) return launch_eval_wide(pm, a, s, (flags & PIB_EVAL_BF16X3) != 0);
   if (a.qf) return launch_eval_fp64_offsets(a.A, a, s);
   return launch_eval_fp64(a.A, a.AR, pm, a, s);

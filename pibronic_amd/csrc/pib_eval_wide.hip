@@ -29,6 +29,7 @@
 // only the leading A x A block, so M is zero outside it; padded surfaces carry O = 0 and drop
 // out of every trace.
 #include "pib_common.hpp"
+#include "pib_expm.hpp"
 #include "pib_kernels.hpp"
 
 namespace pib {
@@ -110,8 +111,6 @@ __device__ __forceinline__ d4 sym_mul(const d4& X, const d4& Y) {
   return sym_mul<NR>(X, Y, d4{0.0, 0.0, 0.0, 0.0});
 }
 
-constexpr double kLog2Theta15 = -0.5640051;  // log2(0.67642)
-
 // exp(X) for a symmetric X in the FP64 accumulator layout, zero outside its leading n x n
 // block, n <= 4 NR: scaling and squaring of the degree-16 polynomial that is the Taylor
 // polynomial through X^15, in four products (the per-lane kernel's form, after Sastre 2018):
@@ -126,14 +125,7 @@ constexpr double kLog2Theta15 = -0.5640051;  // log2(0.67642)
 // result is zero outside it.
 template <int NR>
 __device__ __forceinline__ d4 expm_sym(const d4& X, int n, int g, int j) {
-  constexpr double c1 = -4.01876161020103546293293287596e-4, c2 = -2.94553144027968298047549126357e-3;
-  constexpr double c3 = 8.70906657683767596765346131523e-3, c4 = -4.01756844067356780152362494573e-1;
-  constexpr double c5 = -3.23076288812231208197540935626e-2, c6 = 2.33731940471157926649827413344e-2;
-  constexpr double c7 = 2.61492797729811710806033238185e-1, c8 = -2.38107037387098722469262858218e-1;
-  constexpr double c9 = -4.1302763659297829110328428344e-2, c10 = -5.79236170707326052179805145605e0;
-  constexpr double c11 = 2.22420917249637356119032703879e0, c12 = 1.04080173523135436461532671084e1;
-  constexpr double c13 = 3.03012340073871230596564458406e0, c14 = -2.12975559049643578453357460382e0;
-  constexpr double d3 = c3 - c5, e7 = c7 - c6 * c5, f10 = -c10 * c5, g14 = c14 - c13 * c5;
+  using E = Taylor16;
   const bool dl = ((j & 3) == g) && (j < n);  // register j / 4 of this lane holds X[j][j]
   const int dr = j >> 2;
   const d4 X2 = sym_mul<NR>(X, X);
@@ -143,7 +135,7 @@ __device__ __forceinline__ d4 expm_sym(const d4& X, int n, int g, int j) {
   n2 = wave_sum_dpp(n2);
   // smallest s >= 0 with |X^2|_F^(1/2) 2^-s <= theta_15+; a zero matrix gives -inf, a NaN s = 0,
   // the count is capped at 64
-  const double sd = 0.25 * log2_coarse(n2) - kLog2Theta15;
+  const double sd = 0.25 * log2_coarse(n2) - E::log2_theta;
   int s = 0;
   if (sd > 0.0) s = sd < 64.0 ? (int)ceil(sd) : 64;
   s = __builtin_amdgcn_readfirstlane(s);  // identical on every lane
@@ -152,23 +144,23 @@ __device__ __forceinline__ d4 expm_sym(const d4& X, int n, int g, int j) {
   for (int r = 0; r < 4; ++r) {
     x1[r] = ldexp(X[r], -s);
     x2[r] = ldexp(X2[r], -2 * s);
-    H[r] = fma(c1, x2[r], c2 * x1[r]);
+    H[r] = fma(E::c1, x2[r], E::c2 * x1[r]);
   }
-  const d4 G = sym_mul<NR>(x2, H, c5 * x2);  // y02 + c5 X2
+  const d4 G = sym_mul<NR>(x2, H, E::c5 * x2);  // y02 + E::c5 X2
   d4 F, acc;
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
-    F[r] = fma(c4, x1[r], fma(d3, x2[r], G[r]));  // y02 + c3 X2 + c4 X
-    acc[r] = fma(c6, G[r], e7 * x2[r]);
+    F[r] = fma(E::c4, x1[r], fma(E::d3, x2[r], G[r]));  // y02 + E::c3 X2 + E::c4 X
+    acc[r] = fma(E::c6, G[r], E::e7 * x2[r]);
   }
   const d4 Y = sym_mul<NR>(F, G, acc);  // y12
   d4 F1, F2, R;
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const double I = (dl && r == dr) ? 1.0 : 0.0;
-    F1[r] = fma(c8, x2[r], fma(c9, x1[r], Y[r]));
-    F2[r] = fma(c10, G[r], fma(c11, x1[r], fma(f10, x2[r], Y[r])));
-    R[r] = fma(c12, Y[r], fma(c13, G[r], fma(g14, x2[r], x1[r]))) + I;
+    F1[r] = fma(E::c8, x2[r], fma(E::c9, x1[r], Y[r]));
+    F2[r] = fma(E::c10, G[r], fma(E::c11, x1[r], fma(E::f10, x2[r], Y[r])));
+    R[r] = fma(E::c12, Y[r], fma(E::c13, G[r], fma(E::g14, x2[r], x1[r]))) + I;
   }
   d4 T = sym_mul<NR>(F1, F2, R);
   for (int k = 0; k < s; ++k) T = sym_mul<NR>(T, T);

@@ -40,4 +40,18 @@ struct Exp8 {
   static constexpr double c7 = 0.5000000000000101;
 };
 
+// The degree-16 form with the Taylor polynomial through X^15 (the one-wave-per-sample kernel and its
+// four-sample form), theta_15+ = 0.67642
+struct Taylor16 {
+  static constexpr double c1 = -4.01876161020103546293293287596e-4, c2 = -2.94553144027968298047549126357e-3;
+  static constexpr double c3 = 8.70906657683767596765346131523e-3, c4 = -4.01756844067356780152362494573e-1;
+  static constexpr double c5 = -3.23076288812231208197540935626e-2, c6 = 2.33731940471157926649827413344e-2;
+  static constexpr double c7 = 2.61492797729811710806033238185e-1, c8 = -2.38107037387098722469262858218e-1;
+  static constexpr double c9 = -4.1302763659297829110328428344e-2, c10 = -5.79236170707326052179805145605e0;
+  static constexpr double c11 = 2.22420917249637356119032703879e0, c12 = 1.04080173523135436461532671084e1;
+  static constexpr double c13 = 3.03012340073871230596564458406e0, c14 = -2.12975559049643578453357460382e0;
+  static constexpr double d3 = c3 - c5, e7 = c7 - c6 * c5, f10 = -c10 * c5, g14 = c14 - c13 * c5;
+  static constexpr double log2_theta = -0.5640051;
+};
+
 }  // namespace pib

@@ -245,6 +245,9 @@ hipError_t launch_eval_fp32(int A, int AR, int pm, const EvalArgs& a, hipStream_
 hipError_t launch_eval_batched(int A, int AR, int pm, const LaneProbs& probs, const BatchTile* tiles,
                                int ntiles, int* counter, int waves, hipStream_t s);
 LaneProb lane_prob(const EvalArgs& a);
+// the same results for 9 to 12 surfaces without +-dbeta, four samples per wave
+bool wide4_supported(const EvalArgs& a, int num_cu);
+hipError_t launch_eval_wide4(const EvalArgs& a, hipStream_t s);
 hipError_t launch_eval_wide_batched(int pm, const EvalArgs* probs, const BatchTile* tiles, int ntiles,
                                     int* counter, int waves, hipStream_t s);
 constexpr int kWideMaxStates = 16;
