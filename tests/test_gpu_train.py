@@ -58,3 +58,21 @@ def test_product_stages(tmp_path, ta, tb, K):
     b = (Bm[:, :K].T if tb else Bm[:, :N]).double()
     tol = (3 * 2.0 ** -16 + K * 2.0 ** -24) * (a.abs() @ b.abs())
     assert torch.all((C.cpu().double() - a @ b).abs() <= tol)
+
+
+@pytest.mark.parametrize("N,B", [(16, 82048), (8, 164096)])
+def test_pieces_of_a_large_draw(tmp_path, N, B):
+    """Just beyond the size from which draws are taken in pieces, with a last piece that is no whole
+    launch: draws and offsets are those of the whole batch bit for bit."""
+    print(f"[gpu-case] pieces N={N} B={B}", flush=True)
+    FS = stage_dict_models(tmp_path, random_model(2, N, seed=N))
+    data = make_data(FS, 300.0, 64, 128, 128)
+    fl = flow.Flow(data, layers=3, hidden=256, smax=2.0, gemm="bf16x3")
+    fl.set_params(random_params(ref_for(data, 3, 256, 2.0), 5))
+    fl.draw_precision = "bf16"
+    assert len(fl._chunks(B)) > 1
+    got = [fl.draw(B, 7, 3, offsets=True), fl.draw(B, 7, 3)]
+    fl._chunks = lambda B: [slice(0, B)]
+    want = [fl.draw(B, 7, 3, offsets=True), fl.draw(B, 7, 3)]
+    for g, w in zip(got, want):
+        assert torch.equal(g[0], w[0]) and torch.equal(g[1], w[1])
