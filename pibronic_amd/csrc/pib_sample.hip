@@ -23,8 +23,8 @@
 //
 // Layout: a wave takes one mode of 64 consecutive samples, one lane per row (sample, mode), so
 // the mode's factor entries are wave-uniform scalar loads. Each lane walks its beads
-// downwards in chunks of 8 or 16; a chunk is staged in LDS and the wave then writes the 64 rows'
-// chunk with consecutive lanes on consecutive addresses (64- or 128-byte row segments).
+// downwards in chunks of 8 to 32; a chunk is staged in LDS and the wave then writes the 64 rows'
+// chunk with consecutive lanes on consecutive addresses (64- to 256-byte row segments).
 #include <algorithm>
 
 #include "pib_common.hpp"
@@ -33,13 +33,28 @@
 namespace pib {
 
 constexpr int kSampleWaves = 4;   // waves per work-group, each independent
-// Beads staged per lane before a write-out: 16 (a whole 128-byte line where rows start on one)
-// beyond 24 beads per row, else 8. Half lines written apart reach memory one by one once the rows
-// in flight exceed the L2; short rows lose more by the waves that the larger LDS tile displaces.
-// MI355X, us with 8 / 16, A N P samples: 4 8 64 1e5 122 / 90, 8 16 64 1e5 271 / 160, 6 12 256
-// 16,384 134 / 92, 11 17 50 32,768 74 / 61, 5 7 33 20,000 19.6 / 17.5, 2 6 24 1e5 29 / 33,
-// 3 6 16 1e5 22.0 / 22.8, 2 3 12 1e4 5.6 / 6.3.
-static bool long_rows(const SampleArgs& a) { return a.P > 24; }
+// Beads staged per lane before a write-out: 8 up to 24 beads per row, else 16 (a whole 128-byte line
+// where rows start on one), or 32 where rows start off a line and the launch writes more than the
+// 256 MB of the memory-side cache. Half lines written apart reach memory one by one once the rows in
+// flight exceed the L2, and so do the two ends of a run off the line, fewer in longer runs; short rows
+// and cached writes lose more by the waves that the larger LDS tile displaces. MI355X, us with 8 / 16 / 32,
+// A N P samples: 4 8 64 1e5 122 / 90 / 105, 8 16 64 1e5 271 / 160 / 184, 6 12 256 16,384 134 / 92 / 103,
+// 4 8 101 60,000 206 / 181 / 142, 4 8 60 1e5 (384 MB) 16 / 32: 140 / 126, 6 12 250 16,384 178 / 140,
+// 6 12 70 16,384 (110 MB) 33 / 36, 11 17 50 32,768 74 / 61 / 73; 2 6 24 1e5 29 / 33, 3 6 16 1e5 22.0 / 22.8,
+// 2 3 12 1e4 5.6 / 6.3.
+static int chunk_for(const SampleArgs* a, int n) {
+  double all = 0.0, off = 0.0;
+  int longest = 0;
+  for (int i = 0; i < n; ++i) {
+    const double bytes = 8.0 * a[i].B * a[i].N * a[i].P;
+    const bool line = a[i].P % 16 == 0 && (uintptr_t)a[i].q % 128 == 0;
+    all += bytes;
+    if (!line && a[i].P >= 48) off += bytes;
+    if (a[i].P > longest) longest = a[i].P;
+  }
+  if (longest <= 24) return 8;
+  return all > 256 * 1048576.0 && 2.0 * off > all ? 32 : 16;
+}
 
 __device__ __forceinline__ int draw_source(const SampleArgs& a, int64_t gsample) {
   if (a.A_rho == 1) return 0;
@@ -168,7 +183,7 @@ __global__ void __launch_bounds__(kWave * kSampleWaves) k_sample_fp64(const Samp
 // The samplers of several problems (the temperatures of a batch) in one launch: one problem's
 // rows alone leave the chip mostly waiting on each wave's serial walk over the beads. Sixteen
 // temperatures of A = 6, N = 12, P = 52..256, 16,384 samples each (MI355X): 1.69 ms as sixteen
-// launches with half-line write-out, 1.53 as one with whole lines (3.9 GB written; a fill reaches 6.7 TB/s).
+// launches with half-line write-out, 1.33 as one with 32 beads (3.9 GB written; a fill reaches 6.7 TB/s).
 // The caller puts the longest rows first, so that the short ones fill the tail.
 template <int CHUNK>
 __global__ void __launch_bounds__(kWave * kSampleWaves) k_sample_batched(const SampleBatch b) {
@@ -192,10 +207,12 @@ hipError_t launch_sample_fp64(const SampleArgs& a, hipStream_t s) {
   int64_t groups = (units + kSampleWaves - 1) / kSampleWaves;
   if (groups > 65536) groups = 65536;
   if (groups < 1) groups = 1;
-  if (long_rows(a))
-    hipLaunchKernelGGL(k_sample_fp64<16>, dim3((unsigned)groups), dim3(kWave * kSampleWaves), 0, s, a);
-  else
-    hipLaunchKernelGGL(k_sample_fp64<8>, dim3((unsigned)groups), dim3(kWave * kSampleWaves), 0, s, a);
+  const dim3 grid((unsigned)groups), block(kWave * kSampleWaves);
+  switch (chunk_for(&a, 1)) {
+    case 8: hipLaunchKernelGGL(k_sample_fp64<8>, grid, block, 0, s, a); break;
+    case 16: hipLaunchKernelGGL(k_sample_fp64<16>, grid, block, 0, s, a); break;
+    default: hipLaunchKernelGGL(k_sample_fp64<32>, grid, block, 0, s, a);
+  }
   return hipGetLastError();
 }
 
@@ -204,10 +221,8 @@ hipError_t launch_sample_batch(const SampleArgs* args, int n, hipStream_t s) {
     SampleBatch b{};
     b.n = std::min(kSampleBatchProbs, n - i0);
     int64_t units = 0;
-    bool lng = false;
     for (int i = 0; i < b.n; ++i) {
       b.p[i] = args[i0 + i];
-      lng = lng || long_rows(b.p[i]);
       units += (b.p[i].B + kWave - 1) / kWave * b.p[i].N;
     }
     const int64_t groups = (units + kSampleWaves - 1) / kSampleWaves;
@@ -216,10 +231,12 @@ hipError_t launch_sample_batch(const SampleArgs* args, int n, hipStream_t s) {
         if (hipError_t e = launch_sample_fp64(b.p[i], s)) return e;
       continue;
     }
-    if (lng)
-      hipLaunchKernelGGL(k_sample_batched<16>, dim3((unsigned)groups), dim3(kWave * kSampleWaves), 0, s, b);
-    else
-      hipLaunchKernelGGL(k_sample_batched<8>, dim3((unsigned)groups), dim3(kWave * kSampleWaves), 0, s, b);
+    const dim3 grid((unsigned)groups), block(kWave * kSampleWaves);
+    switch (chunk_for(b.p, b.n)) {
+      case 8: hipLaunchKernelGGL(k_sample_batched<8>, grid, block, 0, s, b); break;
+      case 16: hipLaunchKernelGGL(k_sample_batched<16>, grid, block, 0, s, b); break;
+      default: hipLaunchKernelGGL(k_sample_batched<32>, grid, block, 0, s, b);
+    }
     if (hipError_t e = hipGetLastError()) return e;
   }
   return hipSuccess;

@@ -33,6 +33,24 @@ def test_rows_do_not_depend_on_the_block(tmp_path, P):
         assert torch.all(buf[:lead] == -7.0) and torch.all(buf[lead + B * N * P:] == -7.0)
 
 
+@pytest.mark.parametrize("P", [48, 61, 96, 129])
+def test_long_runs_off_the_line(tmp_path, P):
+    """More than 256 MB of rows off the line (32 beads staged): the draws of smaller launches."""
+    print(f"[gpu-case] sampler long runs P={P}", flush=True)
+    FS = stage_dict_models(tmp_path, random_model(2, 3, seed=P))
+    ctx = make_data(FS, 300.0, P, 100, 100).context()
+    N, lead = 3, 1
+    B = (270 << 20) // (8 * N * P) + 5
+    buf = torch.full((B * N * P + 8,), -7.0, dtype=torch.float64, device=DEV)
+    got = buf[lead:lead + B * N * P].view(B, N, P)
+    ctx.sample_block(9, 5, B, got)
+    part = torch.empty((100, N, P), dtype=torch.float64, device=DEV)
+    for first in (0, 63, B - 100):
+        ctx.sample_block(9, 5 + first, 100, part)
+        assert torch.equal(part, got[first:first + 100]), first
+    assert torch.all(got != -7.0) and buf[0] == -7.0 and torch.all(buf[lead + B * N * P:] == -7.0)
+
+
 @pytest.mark.parametrize("n", [1, 3, 18])
 def test_batched_samplers_and_sums_are_the_single_ones(tmp_path, n):
     """Problems of rising P (one and two launches' worth): draws and sums of every problem and
