@@ -55,6 +55,17 @@ def algorithmic_flops(A, N, P, n_quad_pairs, pm=False):
     return {"sample": sample, "eval": ev, "total": sample + ev}
 
 
+def fp64_kernel_name(A, pm, offsets=False):
+    """The FP64 evaluation kernel of a full-size block with A_rho = A surfaces."""
+    if A >= (7 if pm else 8) and (pm or A == 8):
+        return f"(anonymous namespace)::k_eval_block<{A}, {str(pm).lower()}, {str(offsets).lower()}>"
+    if A > 8:
+        return f"(anonymous namespace)::k_eval_wide4<{A}>" if 9 <= A <= 12 else "k_eval_wide"
+    if offsets:
+        return f"k_eval_fp64_offsets<{A}"
+    return f"k_eval_fp64<{A}, {A}, {str(pm).lower()}, false"
+
+
 def profiled_traffic(path, kernel_prefix):
     """HBM bytes per launch of a kernel from a committed rocprofv3 summary: FETCH_SIZE and
     WRITE_SIZE (KiB per dispatch), each divided by what the same counter reads for a plain
@@ -429,8 +440,7 @@ def pm_leg(FS, cfg, B, steps, W, seed, log, label):
     data = setup_data(FS, cfg, B, steps + W, seed, pm=True)
     h = harmonic_leg(data, B, steps, W, seed, _native.EVAL_PM, True)
     sbs = h["samples"] * P / h["seconds"]
-    kname = ("k_eval_fp64_chain<8, 8, 1..3> (three single-chain passes)" if A == 8
-             else f"k_eval_fp64<{A}, {A}, true, false>" if A <= 8 else "k_eval_wide (+-dbeta)")
+    kname = fp64_kernel_name(A, True)
     log(f"[bench] FP64 +-dbeta {label}: {sbs:.3e} samples*beads/s, eval {h['eval_kernel_ms']:.3f} ms")
     return {"samples_beads_per_s": sbs, "ms_per_step": h["ms_per_step"], "steps": h["steps"], "block": B,
             "eval_kernel_ms": h["eval_kernel_ms"],
@@ -459,9 +469,9 @@ def fp64_line(FS, name, cfg, args, cpu, log):
         torch.cuda.synchronize()
     h = harmonic_leg(data, B, args.fp64_steps, args.warmup, args.seed, 0, False)
     sbs = h["samples"] * P / h["seconds"]
-    kname = f"k_eval_fp64<{A}, {A}, false, false>" if A <= 8 else "k_eval_wide"
-    traffic, tdetail = profiled_traffic(os.path.join(ROOT, "profiles", f"k_eval_fp64_A{A}_N{N}_P{P}_B{B}.md"),
-                                        f"void pib::k_eval_fp64<{A}, {A}, false, false>")
+    kname = fp64_kernel_name(A, False)
+    traffic, tdetail = profiled_traffic(os.path.join(ROOT, "profiles", f"{kname.split('<')[0].split('::')[-1]}_A{A}_N{N}_P{P}_B{B}.md"),
+                                        f"void pib::{kname}")
     log(f"[bench] FP64 {name}: {sbs:.3e} samples*beads/s, eval {h['eval_kernel_ms']:.3f} ms")
     line = {"workload": f"{name}: A={A} N={N} P={P} T={cfg['T']:g}K block={B}, FP64, harmonic rho",
             "samples_beads_per_s": sbs, "samples_per_s": h["samples_per_s"], "ms_per_step": h["ms_per_step"],
@@ -671,7 +681,7 @@ def main():
     harm = harmonic_leg(data, args.block, nblocks, W, args.seed, 0, False)
     log(f"[bench] harmonic {name}: {nblocks} blocks, ess fraction {harm['ess_fraction']:.3e}")
     nq = n_quad_pairs(data)
-    kname = f"k_eval_fp64<{A}, {A}, false, false>" if A <= 8 else "k_eval_wide"
+    kname = fp64_kernel_name(A, False)
     harm_pm = pm_leg(FS, cfg, args.block, max(1, min(nblocks, args.fp64_steps)), W, args.seed + 4, log, name)
 
     learned = fl = None
@@ -691,10 +701,11 @@ def main():
     harm_sbs = harm["samples"] * P / harm["seconds"]
     if learned:
         off = learned.get("coordinates", "").startswith("float offsets")
-        kfull = f"void pib::k_eval_fp64_offsets<{A}>" if off else f"void pib::k_eval_fp64<{A}, {A}, false, false>"
-        roof = eval_roofline(A, N, P, nq, False, B_l, learned["eval_kernel_ms"], kfull[len("void pib::"):],
-                             *profiled_traffic(os.path.join(ROOT, "profiles", f"k_eval_fp64_A{A}_N{N}_P{P}_B{B_l}.md"),
-                                               kfull), coord_bytes=4 if off else 8)
+        kl = fp64_kernel_name(A, False, off)
+        family = "k_eval_block" if A == 8 else "k_eval_fp64"
+        roof = eval_roofline(A, N, P, nq, False, B_l, learned["eval_kernel_ms"], kl,
+                             *profiled_traffic(os.path.join(ROOT, "profiles", f"{family}_A{A}_N{N}_P{P}_B{B_l}.md"),
+                                               f"void pib::{kl}"), coord_bytes=4 if off else 8)
         roof["step_note"] = "the FP64 evaluation of g inside the timed learned step (its largest kernel)"
         value = learned["ess_per_s"]
     else:

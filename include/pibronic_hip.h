@@ -45,8 +45,9 @@ extern "C" {
 /* flags of pib_eval_block */
 #define PIB_EVAL_PM 1      /* also g(beta +- dbeta): block_compute_pm                     */
 #define PIB_EVAL_NOSCALE 2 /* skip the S12 scaling (S_p = 1), as the explicit golden test */
-#define PIB_EVAL_WIDE 4    /* force the one-wave-per-sample kernel (used for A > 8; any
-                              A, A_rho <= 16); a tuning/testing switch, same results       */
+#define PIB_EVAL_WIDE 4    /* force the one-wave-per-sample kernel (any A, A_rho <= 16; without
+                              it small blocks of A > 8 without +-dbeta, and prefactors that
+                              are not positive, take it); a tuning/testing switch           */
 #define PIB_EVAL_FP32 8    /* reduced precision (A <= 8): O-factors, V, M = exp(-tau V) (a
                               scaled and squared Taylor polynomial) and the ring products in
                               FP32 (power-of-two renormalised); FP64 log-scale and rho
@@ -115,8 +116,8 @@ int pib_set_beads(pib_ctx* ctx, int P, double tau);
 /* pib_eval_block for coordinates given as float offsets dq_dev (B*N*P) from the per-mode centre
  * m of pib_flow_set_basis: bead coordinate (s, j, p) = m[j] + (double)dq[(s N + j) P + p],
  * formed in FP64 inside the kernel -- the same doubles pib_flow_whiten(PIB_FLOW_UNWHITEN)
- * writes, so the outputs equal pib_eval_block's on those, bit for bit. The FP64 lanes kernel
- * (A <= 8, A_rho = A) only; flags 0 or PIB_EVAL_NOSCALE. No counterpart in the reference
+ * writes, so the outputs equal pib_eval_block's on those, bit for bit. A <= 8, A_rho = A
+ * only; flags 0 or PIB_EVAL_NOSCALE. No counterpart in the reference
  * (whose coordinates are float64 arrays); for the learned proposal's draws, whose unwhitening
  * then writes and this reads half the bytes. */
 int pib_eval_block_flow_offsets(pib_ctx* ctx, const float* dq_dev, int64_t B, int flags, double* out_dev,

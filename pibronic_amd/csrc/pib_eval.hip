@@ -682,6 +682,14 @@ k_eval_batched(const LaneProbs probs, const BatchTile* __restrict__ tiles, int n
 }
 
 // ---------------------------------------------------------------------------------------
+// Sizes with folded instances: up to four surfaces. MI355X, us, general / folded, A N P samples: 2 10 40 1e5
+// 116.5 / 109.5, 3 10 40 1e5 149 / 143 and with +-dbeta 239 / 201, 4 8 64 1e5 267 / 258 and 402 / 391; the
+// wider ones lose by their schedule what the exponents save: 5 17 56 4,000 39 / 46, 5 10 64 1e5
+// 433 / 426 and 902 / 929, 6 12 64 3,000 39.2 / 40.5 and 1e5 1,383 / 1,410 with +-dbeta, 7 14 64 1e5
+// 1,176 / 1,211.
+template <int A, int AR>
+constexpr bool folds = A == AR && A <= 4;
+
 template <int A, int AR>
 static hipError_t launch_a(int pm, const EvalArgs& a, hipStream_t s) {
   const int spw = kWave / a.G;
@@ -701,8 +709,8 @@ static hipError_t launch_a(int pm, const EvalArgs& a, hipStream_t s) {
     if constexpr (A < 7) {
       if (dbg)
         hipLaunchKernelGGL((k_eval_fp64<A, AR, true, true>), grid, dim3(threads), lds, s, b);
-      else if (A == AR && a.fold)
-        hipLaunchKernelGGL((k_eval_fp64<A, AR, true, false, A == AR>), grid, dim3(threads), lds, s, b);
+      else if (folds<A, AR> && a.fold)
+        hipLaunchKernelGGL((k_eval_fp64<A, AR, true, false, folds<A, AR>>), grid, dim3(threads), lds, s, b);
       else
         hipLaunchKernelGGL((k_eval_fp64<A, AR, true, false>), grid, dim3(threads), lds, s, b);
     } else {
@@ -710,8 +718,8 @@ static hipError_t launch_a(int pm, const EvalArgs& a, hipStream_t s) {
     }
   } else if (dbg)
     hipLaunchKernelGGL((k_eval_fp64<A, AR, false, true>), grid, dim3(threads), lds, s, b);
-  else if (A == AR && a.fold)
-    hipLaunchKernelGGL((k_eval_fp64<A, AR, false, false, A == AR>), grid, dim3(threads), lds, s, b);
+  else if (folds<A, AR> && a.fold)
+    hipLaunchKernelGGL((k_eval_fp64<A, AR, false, false, folds<A, AR>>), grid, dim3(threads), lds, s, b);
   else
     hipLaunchKernelGGL((k_eval_fp64<A, AR, false, false>), grid, dim3(threads), lds, s, b);
   return hipGetLastError();
@@ -721,6 +729,7 @@ template <int A, int AR>
 static hipError_t launch_batched_a(int pm, const LaneProbs& probs, const BatchTile* tiles, int ntiles,
                                    int* counter, int waves, hipStream_t s) {
   const dim3 grid((unsigned)((waves + 3) / 4));
+  // the persistent kernel gains by folding at every size (sixteen temperatures of A = 6, us: 3,943 / 3,855)
   const bool fold = A == AR && probs.fold;
   if (pm && fold)
     hipLaunchKernelGGL((k_eval_batched<A, AR, true, A == AR>), grid, dim3(256), 0, s, probs, tiles, ntiles, counter);
@@ -760,8 +769,8 @@ static hipError_t launch_offsets_a(const EvalArgs& a, hipStream_t s) {
   const int64_t waves = (a.B + spw - 1) / spw;
   const int threads = 256;
   const dim3 grid((unsigned)((waves * kWave + threads - 1) / threads));
-  if (a.fold)
-    hipLaunchKernelGGL((k_eval_fp64_offsets<A, true>), grid, dim3(threads), 0, s, a);
+  if (folds<A, A> && a.fold)
+    hipLaunchKernelGGL((k_eval_fp64_offsets<A, folds<A, A>>), grid, dim3(threads), 0, s, a);
   else
     hipLaunchKernelGGL((k_eval_fp64_offsets<A, false>), grid, dim3(threads), 0, s, a);
   return hipGetLastError();
