@@ -111,17 +111,24 @@ int rebuild_block_table(pib_ctx* c) {
 }
 
 // The block kernel takes every (A, A_rho) without a lanes kernel (without +-dbeta up to eight
-// surfaces), and of those with one the sizes where it is the faster: A = 8, and with +-dbeta
-// (three ring chains in one lane's registers) A = 7. Measured (MI355X, us, lanes / block, N = 2 A, P = 64): A = 8 1,000 samples 46 / 27, 16,384
-// 388 / 237, 1e5 1650 / 1416; with +-dbeta 1e5 5470 / 1882; A = 7 1e5 1219 / 1290, with +-dbeta
-// 16,384 837 / 286, 1e5 3163 / 1706; A = 6 1e5 732 / 1235, with +-dbeta 1458 / 1595.
-bool uses_block(const pib_ctx* c, int flags) {
+// surfaces), and of those with one the sizes where it is the faster: A = 8, with +-dbeta (three ring
+// chains in one lane's registers) A = 7, and below certain batches, where lanes kernels of one or two
+// waves per SIMD leave the chip waiting, A = 7 (256 samples per CU) and with +-dbeta A = 6 (256) and A = 5
+// (128), unless the caller has set the lanes per sample. Measured (MI355X, us, lanes / block, N = 2 A, P = 64):
+// A = 8 1,000 samples 46 / 27, 16,384 388 / 237, 1e5 1650 / 1416; with +-dbeta 1e5 5470 / 1882; A = 7
+// 700 33 / 23, 8,000 207 / 108, 64,000 798 / 780, 1e5 1179 / 1290, with +-dbeta 16,384 837 / 286, 1e5
+// 3163 / 1706; A = 6 3,000 39 / 43, 1e5 732 / 1235, with +-dbeta 700 47 / 26, 16,000 563 / 261, 64,000
+// 1286 / 982, 80,000 1115 / 1220; A = 5 3,000 29 / 38, with +-dbeta 700 29 / 24, 32,000 702 / 452, 45,000
+// 573 / 616.
+bool uses_block(const pib_ctx* c, int flags, int64_t B) {
   const bool pm = (flags & PIB_EVAL_PM) != 0;
   if (!c->block_ok[pm] || (flags & (PIB_EVAL_WIDE | PIB_EVAL_FP32 | PIB_EVAL_BF16X3))) return false;
   for (int s = 0; s < (pm ? 4 : 2); ++s)
     if (!c->pref_positive[s]) return false;  // it works with log F_a
   if (!eval_supported(c->A, c->set_A[SET_RHO])) return pm || block_size(c->A, c->set_A[SET_RHO]) <= 8;
-  return c->A >= (pm ? 7 : 8);
+  if (c->A >= (pm ? 7 : 8)) return true;
+  if (c->lanes) return false;
+  return B <= (int64_t)c->num_cu * (c->A == (pm ? 6 : 7) ? 256 : pm && c->A == 5 ? 128 : 0);
 }
 
 // Bead streams per sample (1, 2 or 4) of the block kernel: more of them fill the chip with fewer
@@ -185,7 +192,8 @@ static BlockArgs block_args(const pib_ctx* c, const EvalArgs& a, bool pm) {
 hipError_t launch_eval(const pib_ctx* c, int flags, bool wide, const EvalArgs& a, hipStream_t s) {
   const int pm = (flags & PIB_EVAL_PM) ? 1 : 0;
   if (flags & PIB_EVAL_FP32) return launch_eval_fp32(a.A, a.AR, pm, a, s);
-  if (uses_block(c, flags)) return launch_eval_block(pm, block_args(c, a, pm != 0), s);
+  // offsets: the block kernel has them at A = 8
+  if (uses_block(c, flags, a.B) && (!a.qf || c->A == 8)) return launch_eval_block(pm, block_args(c, a, pm != 0), s);
   if (wide && !pm && !(flags & (PIB_EVAL_WIDE | PIB_EVAL_BF16X3)) && wide4_supported(a, c->num_cu))
     return launch_eval_wide4(a, s);
   if (wide) return launch_eval_wide(pm, a, s, (flags & PIB_EVAL_BF16X3) != 0);

@@ -184,3 +184,28 @@ def test_batch_runs_them_one_launch_each(tmp_path):
         single = pimc.evaluate_samples(d, q, pm=True)
         for k in KEYS_PM + ["log_scale"]:
             assert np.array_equal(res[k], single[k]), k
+
+
+@pytest.mark.parametrize("A,pm,P", [(5, True, 7), (6, True, 9), (7, False, 6)])
+def test_small_batches_of_lanes_sizes(tmp_path, A, pm, P):
+    """Sizes with a lanes kernel that small batches take to the block kernel: both against each other
+    on the same samples (set lanes per sample keep the lanes kernel), and the larger batch that stays
+    with the lanes kernel, bit for bit what its own lanes give."""
+    _announce(f"block small batches A={A} pm={pm}")
+    FS = stage_dict_models(tmp_path, random_model(A, 2, seed=A, quad="full"))
+    data = make_data(FS, 300.0, P, 300, 300, pm=pm)
+    q, _ = data.draw_host_sample(np.random.default_rng(A), 300)
+    keys = KEYS_PM if pm else KEYS
+    block = pimc.evaluate_samples(data, q, pm=pm)
+    _close(block, po.evaluate(oracle_setup(FS, 300.0, P), q, pm=pm), keys, 1e-10)
+    ctx = data.context()
+    ctx.set_lanes_per_sample(4)
+    lanes = pimc.evaluate_samples(data, q, pm=pm)
+    _close(block, lanes, keys, 1e-11)
+    big = np.concatenate([q] * 220)  # 66,000 samples
+    a = pimc.evaluate_samples(data, big, pm=pm)
+    ctx.set_lanes_per_sample(ctx.lanes_per_sample(len(big)))
+    b = pimc.evaluate_samples(data, big, pm=pm)
+    for k in keys:
+        assert np.array_equal(a[k], b[k]), k
+        assert np.array_equal(a[k][:300], lanes[k]), k
