@@ -113,10 +113,11 @@ int rebuild_block_table(pib_ctx* c) {
 // The block kernel takes every (A, A_rho) without a lanes kernel (without +-dbeta up to eight
 // surfaces), and of those with one the sizes where it is the faster: A = 8, with +-dbeta (three ring
 // chains in one lane's registers) A = 7, and below certain batches, where lanes kernels of one or two
-// waves per SIMD leave the chip waiting, A = 7 (256 samples per CU) and with +-dbeta A = 6 (256) and A = 5
+// waves per SIMD leave the chip waiting, A = 7 (160 samples per CU) and with +-dbeta A = 6 (256) and A = 5
 // (128), unless the caller has set the lanes per sample. Measured (MI355X, us, lanes / block, N = 2 A, P = 64):
 // A = 8 1,000 samples 46 / 27, 16,384 388 / 237, 1e5 1650 / 1416; with +-dbeta 1e5 5470 / 1882; A = 7
-// 700 33 / 23, 8,000 207 / 108, 64,000 798 / 780, 1e5 1179 / 1290, with +-dbeta 16,384 837 / 286, 1e5
+// 700 33 / 23, 8,000 207 / 108, 32,000 501 / 397, 64,000 798 / 780 (N = 3, 47,000 block step 464 / 470), 1e5
+// 1179 / 1290, with +-dbeta 16,384 837 / 286, 1e5
 // 3163 / 1706; A = 6 3,000 39 / 43, 1e5 732 / 1235, with +-dbeta 700 47 / 26, 16,000 563 / 261, 64,000
 // 1286 / 982, 80,000 1115 / 1220; A = 5 3,000 29 / 38, with +-dbeta 700 29 / 24, 32,000 702 / 452, 45,000
 // 573 / 616.
@@ -128,7 +129,7 @@ bool uses_block(const pib_ctx* c, int flags, int64_t B) {
   if (!eval_supported(c->A, c->set_A[SET_RHO])) return pm || block_size(c->A, c->set_A[SET_RHO]) <= 8;
   if (c->A >= (pm ? 7 : 8)) return true;
   if (c->lanes) return false;
-  return B <= (int64_t)c->num_cu * (c->A == (pm ? 6 : 7) ? 256 : pm && c->A == 5 ? 128 : 0);
+  return B <= (int64_t)c->num_cu * (pm ? (c->A == 6 ? 256 : c->A == 5 ? 128 : 0) : (c->A == 7 ? 160 : 0));
 }
 
 // Bead streams per sample (1, 2 or 4) of the block kernel: more of them fill the chip with fewer
