@@ -108,13 +108,6 @@ __device__ __forceinline__ float dpp_f(float x) {
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(u, u, CTRL, 0xF, 0xF, false));
 }
 
-// a constant times 2^-k, k wave-uniform: an exponent adjustment on the scalar unit
-__device__ __forceinline__ double down(double c, int k) {
-  const unsigned long long u = __builtin_bit_cast(unsigned long long, c);
-  const unsigned hi = (unsigned)(u >> 32) - ((unsigned)k << 20);
-  return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | (unsigned)u);
-}
-
 // Z = X Y + Z for commuting symmetric X, Y and a symmetric Z given by its blocks I <= K
 template <int NB>
 __device__ __forceinline__ void sym_mul_upper(const double (&X)[NB][NB], const double (&Y)[NB][NB],
@@ -145,12 +138,17 @@ __device__ __forceinline__ void sym_mul(const double (&X)[NB][NB], const double 
   mirror<NB>(Z, ident);
 }
 
-// T = exp(X) of the wave's four symmetric matrices, zero outside the leading n x n block: Exp16's
-// degree-16 polynomial in four products, scaled and squared. One squaring count for the four
-// matrices, so the scaling by 2^-s goes into the (scalar) coefficients instead of X and X^2.
-// alpha = |X^2|_F^(1/2) needs only its binary exponent: its sum is taken in FP32.
+// T = exp(X) of the wave's four symmetric matrices, zero outside the leading n x n block (X is
+// scaled in place): Exp16's degree-16 polynomial in four products, scaled and squared. Each stream has
+// its own scaling 2^-s and is squared s times (powers of two are exact), so that its bits are the same
+// whichever samples share the wave; the wave runs the largest count. One count for all four costs less
+// (A = 11, N = 17, P = 50, 3,001 samples with +-dbeta 128 / 133 us, A = 8 the same) and loses up to all
+// digits of a sample beside one whose |tau V| is large. Scaling the coefficients on the scalar unit
+// where the counts agree is slower (A = 8, N = 16, P = 64, 1e5 samples with +-dbeta 1,793 / 1,816 us).
+// alpha = |X^2|_F^(1/2) needs only its binary exponent: its sum is taken in FP32, of alpha^4 2^-100
+// (alpha up to 2^57 without overflow; below 2^-6, where s is 0 anyway, it may vanish).
 template <int NB>
-__device__ __forceinline__ void expm_block(const double (&X)[NB][NB], int n, int i, int j, double ident,
+__device__ __forceinline__ void expm_block(double (&X)[NB][NB], int n, int i, int j, double ident,
                                            double (&T)[NB][NB]) {
   using E = Exp16;
   double X2[NB][NB], G[NB][NB], F[NB][NB];
@@ -162,7 +160,7 @@ __device__ __forceinline__ void expm_block(const double (&X)[NB][NB], int n, int
 #pragma unroll
     for (int K = I + 1; K < NB; ++K) no = fma(X2[I][K], X2[I][K], no);
   }
-  float m = (float)fma(2.0, no, nd);
+  float m = (float)fma(0x1p-99, no, 0x1p-100 * nd);
   m += dpp_f<0xB1>(m);  // over the four columns of the stream: quad_perm [1,0,3,2], [2,3,0,1]
   m += dpp_f<0x4E>(m);
   {  // over the four rows
@@ -173,62 +171,63 @@ __device__ __forceinline__ void expm_block(const double (&X)[NB][NB], int n, int
     r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
     m = __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
   }
-  m = fmaxf(m, dpp_f<0x124>(m));  // the largest of the four streams: row_ror 4, 8
-  m = fmaxf(m, dpp_f<0x128>(m));
   // smallest s >= 0 with alpha 2^-s <= theta; a zero matrix gives -inf, a NaN s = 0
-  const float sd = 0.25f * __log2f(m) - (float)E::log2_theta;
+  const float sd = fmaf(0.25f, __log2f(m), 25.0f - (float)E::log2_theta);
   int s = 0;
   if (sd > 0.0f) s = sd < 64.0f ? (int)ceilf(sd) : 64;
-  s = __builtin_amdgcn_readfirstlane(s);
-  {
-    const double k1 = down(E::c1, 4 * s), k2 = down(E::c2, 3 * s), k5 = down(E::c5, 2 * s);
+  int smax = max(s, __builtin_amdgcn_update_dpp(s, s, 0x124, 0xF, 0xF, false));  // the streams: row_ror 4, 8
+  smax = max(smax, __builtin_amdgcn_update_dpp(smax, smax, 0x128, 0xF, 0xF, false));
+  smax = __builtin_amdgcn_readfirstlane(smax);
+  if (smax) {
+    const double k1 = __builtin_bit_cast(double, (unsigned long long)(1023 - s) << 52), k2 = k1 * k1;
 #pragma unroll
     for (int I = 0; I < NB; ++I)
 #pragma unroll
       for (int K = 0; K < NB; ++K) {
-        F[I][K] = fma(k1, X2[I][K], k2 * X[I][K]);
-        if (K >= I) G[I][K] = k5 * X2[I][K];
+        X[I][K] *= k1;
+        X2[I][K] *= k2;
       }
   }
+#pragma unroll
+  for (int I = 0; I < NB; ++I)
+#pragma unroll
+    for (int K = 0; K < NB; ++K) {
+      F[I][K] = fma(E::c1, X2[I][K], E::c2 * X[I][K]);
+      if (K >= I) G[I][K] = E::c5 * X2[I][K];
+    }
   sym_mul_upper<NB>(X2, F, G);  // G = y02 + c5 X2
   mirror<NB>(G, ident);
-  {
-    const double k3 = down(E::d3, 2 * s), k4 = down(E::c4, s), k7 = down(E::e7, 2 * s);
 #pragma unroll
-    for (int I = 0; I < NB; ++I)
+  for (int I = 0; I < NB; ++I)
 #pragma unroll
-      for (int K = 0; K < NB; ++K) {
-        F[I][K] = fma(k4, X[I][K], fma(k3, X2[I][K], G[I][K]));
-        if (K >= I) T[I][K] = fma(E::c6, G[I][K], k7 * X2[I][K]);
-      }
-  }
+    for (int K = 0; K < NB; ++K) {
+      F[I][K] = fma(E::c4, X[I][K], fma(E::d3, X2[I][K], G[I][K]));
+      if (K >= I) T[I][K] = fma(E::c6, G[I][K], E::e7 * X2[I][K]);
+    }
   sym_mul_upper<NB>(F, G, T);  // T = y12
   mirror<NB>(T, ident);
-  {
-    const double k8 = down(E::c8, 2 * s), k9 = down(E::c9, s), k11 = down(E::c11, s), k10 = down(E::f10, 2 * s);
-    const double k14 = down(E::g14, 2 * s), kx = down(1.0, s);
 #pragma unroll
-    for (int I = 0; I < NB; ++I)
+  for (int I = 0; I < NB; ++I)
 #pragma unroll
-      for (int K = 0; K < NB; ++K) {
-        const double x = X[I][K], x2 = X2[I][K], gg = G[I][K], y = T[I][K];
-        F[I][K] = fma(k8, x2, fma(k9, x, y));
-        G[I][K] = fma(E::c10, gg, fma(k11, x, fma(k10, x2, y)));
-        if (K >= I) {
-          double r = fma(E::c12, y, fma(E::c13, gg, fma(k14, x2, kx * x)));
-          if (K == I) r += (i == j && 4 * I + i < n) ? 1.0 : 0.0;
-          T[I][K] = r;
-        }
+    for (int K = 0; K < NB; ++K) {
+      const double x = X[I][K], x2 = X2[I][K], gg = G[I][K], y = T[I][K];
+      F[I][K] = fma(E::c8, x2, fma(E::c9, x, y));
+      G[I][K] = fma(E::c10, gg, fma(E::c11, x, fma(E::f10, x2, y)));
+      if (K >= I) {
+        double r = fma(E::c12, y, fma(E::c13, gg, fma(E::g14, x2, x)));
+        if (K == I) r += (i == j && 4 * I + i < n) ? 1.0 : 0.0;
+        T[I][K] = r;
       }
-  }
+    }
   sym_mul_upper<NB>(F, G, T);
   mirror<NB>(T, ident);
-  for (int k = 0; k < s; ++k) {
+  for (int k = 0; k < smax; ++k) {
     sym_mul<NB>(T, T, ident, F);
+    const bool mine = k < s;
 #pragma unroll
     for (int I = 0; I < NB; ++I)
 #pragma unroll
-      for (int K = 0; K < NB; ++K) T[I][K] = F[I][K];
+      for (int K = 0; K < NB; ++K) T[I][K] = mine ? F[I][K] : T[I][K];
   }
 }
 
