@@ -193,8 +193,7 @@ static BlockArgs block_args(const pib_ctx* c, const EvalArgs& a, bool pm) {
 hipError_t launch_eval(const pib_ctx* c, int flags, bool wide, const EvalArgs& a, hipStream_t s) {
   const int pm = (flags & PIB_EVAL_PM) ? 1 : 0;
   if (flags & PIB_EVAL_FP32) return launch_eval_fp32(a.A, a.AR, pm, a, s);
-  // offsets: the block kernel has them at A = 8
-  if (uses_block(c, flags, a.B) && (!a.qf || c->A == 8)) return launch_eval_block(pm, block_args(c, a, pm != 0), s);
+  if (uses_block(c, flags, a.B)) return launch_eval_block(pm, block_args(c, a, pm != 0), s);
   if (wide && !pm && !(flags & (PIB_EVAL_WIDE | PIB_EVAL_BF16X3)) && wide4_supported(a, c->num_cu))
     return launch_eval_wide4(a, s);
   if (wide) return launch_eval_wide(pm, a, s, (flags & PIB_EVAL_BF16X3) != 0);

@@ -536,7 +536,7 @@ hipError_t launch_s(int pm, const BlockArgs& a, hipStream_t s) {
   const int spw = 4 / a.C;
   const dim3 grid((unsigned)((a.B + spw - 1) / spw));
   if (a.qf) {
-    if constexpr (S == 8) {
+    if constexpr (S == 7 || S == 8) {
       if (pm) return hipErrorInvalidValue;
       hipLaunchKernelGGL((k_eval_block<S, false, true>), grid, dim3(kWave), 0, s, a);
     } else {
