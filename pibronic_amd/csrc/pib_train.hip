@@ -433,7 +433,9 @@ __global__ void __launch_bounds__(64 * kTrainWaves) k_train_backward(TrainArgs a
 // 128 x 128 of all pairs in one grid, each wave 64 x 32 of it (12 LDS reads per 24 matrix
 // instructions). K = samples in stages of 32, two in LDS; a thread converts 8 consecutive samples of
 // one column, so reads are coalesced rows and LDS takes 16-byte writes. M and N are multiples of 64:
-// the half tile past the edge repeats the last column and is not stored.
+// the half tile past the edge repeats the last column and is not stored. Every kWeightPart samples the
+// accumulators go into a second sum: the matrix unit's rounding errors of one chain grow with the
+// square of its length (32,768 equal samples: 2.1e-4 of the sum in one chain, 2.4e-6 so; the launch costs the same).
 constexpr int kWeightProbs = 24;
 struct WeightProb {
   const float* X;   // rows x M
@@ -448,7 +450,7 @@ struct WeightArgs {
   int64_t rows;
   WeightProb p[kWeightProbs];
 };
-constexpr int kWTile = 128, kWRow = 32 + 8;
+constexpr int kWTile = 128, kWRow = 32 + 8, kWeightPart = 256;
 struct WeightStage {
   unsigned short Xh[kWTile][kWRow], Xl[kWTile][kWRow], Yh[kWTile][kWRow], Yl[kWTile][kWRow];
 };
@@ -494,11 +496,20 @@ __global__ void __launch_bounds__(512) k_weight_grads(WeightArgs a) {
       bs += u;
     }
   };
-  f32x4t acc[4][2];
+  f32x4t acc[4][2], total[4][2];
 #pragma unroll
   for (int x = 0; x < 4; ++x)
 #pragma unroll
-    for (int y = 0; y < 2; ++y) acc[x][y] = f32x4t{0.f, 0.f, 0.f, 0.f};
+    for (int y = 0; y < 2; ++y) acc[x][y] = total[x][y] = f32x4t{0.f, 0.f, 0.f, 0.f};
+  auto part = [&]() {
+#pragma unroll
+    for (int x = 0; x < 4; ++x)
+#pragma unroll
+      for (int y = 0; y < 2; ++y) {
+        total[x][y] += acc[x][y];
+        acc[x][y] = f32x4t{0.f, 0.f, 0.f, 0.f};
+      }
+  };
   load(0);
   put(st[0]);
   __syncthreads();
@@ -528,8 +539,10 @@ __global__ void __launch_bounds__(512) k_weight_grads(WeightArgs a) {
       for (int y = 0; y < 2; ++y) acc[x][y] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xh, yh[y], acc[x][y], 0, 0, 0);
     }
     if (more) put(st[b ^ 1]);
+    if ((k0 + 32) % kWeightPart == 0) part();  // uniform
     __syncthreads();
   }
+  part();
 #pragma unroll
   for (int x = 0; x < 4; ++x)
 #pragma unroll
@@ -537,7 +550,7 @@ __global__ void __launch_bounds__(512) k_weight_grads(WeightArgs a) {
       const int col = n0 + wc * 32 + y * 16 + (lane & 15), row = m0 + wr * 64 + x * 16 + 4 * (lane >> 4);
       if (col < p.N && row < p.M)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) p.dW[(int64_t)(row + r) * p.N + col] = acc[x][y][r];
+        for (int r = 0; r < 4; ++r) p.dW[(int64_t)(row + r) * p.N + col] = total[x][y][r];
     }
   if (!sum) return;  // uniform
   double* sh = (double*)wlds;
