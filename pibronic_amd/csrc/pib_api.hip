@@ -19,10 +19,11 @@ namespace pib {
 
 // Per-mode constant records of the lanes kernel (layout: ModeRec). Rebuilt by the coupling
 // and O-matrix set setters once the coupling and the rho and vib sets agree in shape; the
-// +-dbeta entries stay zero until those sets are given.
+// +-dbeta entries stay zero until those sets are given. pm_only: only a +-dbeta set has changed.
 int rebuild_block_table(pib_ctx* c);
-int rebuild_mode_table(pib_ctx* c) {
-  c->mode_tab_ok = c->block_ok[0] = c->block_ok[1] = false;
+int rebuild_mode_table(pib_ctx* c, bool pm_only = false) {
+  c->mode_tab_ok = c->block_ok[1] = false;
+  if (!pm_only) c->block_ok[0] = false;
   const int A = c->A, N = c->N, AR = c->set_A[SET_RHO];
   if (!c->coupling_set || !AR || c->set_A[SET_VIB] != A || c->set_N[SET_RHO] != N || c->set_N[SET_VIB] != N)
     return PIB_OK;
@@ -77,18 +78,16 @@ int rebuild_mode_table(pib_ctx* c) {
   return rebuild_block_table(c);
 }
 
-// Constants of the block kernel, rebuilt by the setters once the coupling, the rho and vib sets
-// and the beads agree (in the usual order of calls once, when the beads are set).
+// Constants of the block kernel, rebuilt with the mode table (free of P and tau: the beads may be set
+// while launches are queued or captured).
 int rebuild_block_table(pib_ctx* c) {
-  c->block_ok[0] = c->block_ok[1] = false;
   const int A = c->A, N = c->N, AR = c->set_A[SET_RHO];
-  if (!c->mode_tab_ok || c->P < 3 || A > kWideMaxStates || AR > kWideMaxStates) return PIB_OK;
+  if (A > kWideMaxStates || AR > kWideMaxStates) return PIB_OK;
   if (A < 5 && eval_supported(A, AR)) return PIB_OK;  // never routed to the block kernel
   BlockModel m{};
   m.A = A;
   m.AR = AR;
   m.N = N;
-  m.tau = c->tau;
   m.energy = c->h_energy.data();
   m.linear = c->h_linear.data();
   m.qdiag = c->h_qdiag.empty() ? nullptr : c->h_qdiag.data();
@@ -100,6 +99,7 @@ int rebuild_block_table(pib_ctx* c) {
       m.set[s] = {c->set_A[s],         c->h_th[s].data(), c->h_cs[s].data(),
                   c->h_lin[s].data(), c->h_k2[s].data(), c->h_lpref[s].data()};
     }
+    if (c->block_ok[pm]) continue;
     BlockTables& t = c->block[pm];
     t = block_tables(m, pm != 0);
     const int r = upload(c, c->block_tab[pm], t.data.data(), t.data.size() * sizeof(double));
@@ -172,6 +172,7 @@ static BlockArgs block_args(const pib_ctx* c, const EvalArgs& a, bool pm) {
   b.C = block_streams(c->num_cu, a.B, a.P);
   b.K = (a.P + b.C - 1) / b.C;
   b.noscale = a.noscale;
+  b.ntau = -a.tau;
   b.quad = a.qdiag != nullptr;
   b.npair = a.npair;
   b.ldiag = k.ldiag;
@@ -512,7 +513,7 @@ int pib_set_omatrix_set(pib_ctx* c, int slot, int A_set, int N, const double* co
   }
   c->set_A[slot] = A_set;
   c->set_N[slot] = N;
-  return rebuild_mode_table(c);
+  return rebuild_mode_table(c, slot == SET_VIB_PLUS || slot == SET_VIB_MINUS);
 }
 
 int pib_set_beads(pib_ctx* c, int P, double tau) {
@@ -522,7 +523,7 @@ int pib_set_beads(pib_ctx* c, int P, double tau) {
   if (!std::isfinite(tau) || tau <= 0.0) return fail(c, PIB_ERR_ARG, "set_beads: tau must be > 0");
   c->P = P;
   c->tau = tau;
-  return rebuild_block_table(c);
+  return PIB_OK;
 }
 
 int pib_set_lanes_per_sample(pib_ctx* c, int lanes) {

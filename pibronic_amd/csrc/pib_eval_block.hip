@@ -403,7 +403,7 @@ k_eval_block(const BlockArgs a) {
 #pragma unroll
     for (int q = 0; q < NT; ++q)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) ldsV[(16 * q + row + 4 * r) * Z::ldx + n] = v[q][r];
+      for (int r = 0; r < 4; ++r) ldsV[(16 * q + row + 4 * r) * Z::ldx + n] = a.ntau * v[q][r];
     // O-factors in the log domain (surface 4 I + row of bead n in register I of a set), S_p = max
     // over both models' (pimc.py:1076-1084)
     double lo[NQ], lS = -INFINITY;
@@ -599,15 +599,15 @@ BlockTables block_tables(const BlockModel& m, bool pm) {
     for (int c = 0; c <= r; ++c) {
       const int id = r == c ? S * (S - 1) / 2 + r : r * (r - 1) / 2 + c, q = id / 16, e = id % 16;
       const size_t el = (size_t)r * m.A + c;
-      d[t.energy + 16 * q + 4 * (e % 4) + e / 4] = -m.tau * m.energy[el];
+      d[t.energy + 16 * q + 4 * (e % 4) + e / 4] = m.energy[el];
       for (int j = 0; j < m.N; ++j) {
         const double L = m.linear[j * AA + el];
-        op(j, q < NTL ? NL + q : NL + NT + q, e) = -m.tau * L;
+        op(j, q < NTL ? NL + q : NL + NT + q, e) = L;
         if (q >= NTL && L != 0.0) t.ldiag = 1;
-        if (m.qdiag) op(j, NL + NTL + q, e) = -m.tau * m.qdiag[j * AA + el];
+        if (m.qdiag) op(j, NL + NTL + q, e) = m.qdiag[j * AA + el];
       }
       for (int k = 0; k < npair; ++k)
-        d[t.cpair + ((size_t)(k / 4) * NT + q) * 64 + 16 * (k % 4) + e] = -m.tau * m.qpair[k * AA + el];
+        d[t.cpair + ((size_t)(k / 4) * NT + q) * 64 + 16 * (k % 4) + e] = m.qpair[k * AA + el];
     }
   for (int s = 0; s < sets; ++s) {
     const BlockModel::Set& st = m.set[s];

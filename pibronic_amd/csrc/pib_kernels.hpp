@@ -200,17 +200,18 @@ struct BlockArgs {
   int S;                // the kernel's size, block_size(A, AR)
   int C, K;             // bead streams per sample (1, 2, 4), beads per stream = ceil(P / C)
   int noscale, quad, npair;
+  double ntau;          // -tau
   int ldiag;            // the linear couplings have elements beyond the off-diagonal tiles
   int op_pairs;         // operand pairs per mode group
   const int* pair;
-  const double* energy;  // [tile][e % 4][e / 4], e the element's row in its tile; times -tau
+  const double* energy;  // [tile][e % 4][e / 4], e the element's row in its tile
   const double* k2;      // [register / 4][surface % 4][register % 4]
   const double* lpref;   // the same; -inf for padded surfaces
   const double* tcs;     // [mode][4 sets]{th, csch}
   const double* ops;     // [mode / 4][operand / 2][16 (mode % 4) + row][operand % 2]; operands: the
                          // O-exponents' linear parts (row 4 (register % 4) + surface % 4), linear and
-                         // quadratic couplings (row e), the rest of the linear ones; times -tau
-  const double* cpair;   // [pair / 4][tile][16 (pair % 4) + e], times -tau
+                         // quadratic couplings (row e), the rest of the linear ones
+  const double* cpair;   // [pair / 4][tile][16 (pair % 4) + e]
   double* out;
   int64_t out_stride;
   double* dbg;
@@ -224,7 +225,6 @@ hipError_t launch_eval_block(int pm, const BlockArgs& a, hipStream_t s);
 // Host model the block kernel's constants are built from.
 struct BlockModel {
   int A, AR, N;
-  double tau;
   const double* energy;  // A*A
   const double* linear;  // N*A*A
   const double* qdiag;   // N*A*A = 0.5*Q[j,j] or nullptr
