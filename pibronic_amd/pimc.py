@@ -621,6 +621,10 @@ class BoxResultPM(BoxResult):
 # --------------------------------------------------------------------------------------
 # block loops
 # --------------------------------------------------------------------------------------
+#: what a block is made of, as this module defines it
+_BLOCK_STEPS = {name: getattr(BoxData, name) for name in ("draw_sample", "draw_host_sample", "evaluate_device")}
+
+
 def _run_blocks(data, result, pm):
     import torch
     assert data.blocks * data.block_size <= result.samples, "result is smaller than the run"
@@ -647,33 +651,42 @@ def _run_blocks(data, result, pm):
     host = data.host_buffers(B, min(2, data.blocks))
     views = host.numpy()
     copied = [torch.cuda.Event() for _ in range(host.shape[0])]
+    # Steps of the caller's own (a subclass, an attribute) may use other streams, which know nothing of the
+    # block before, or read the result so far: each block is then collected before the next is drawn.
+    own = any(getattr(getattr(data, name), "__func__", None) is not f for name, f in _BLOCK_STEPS.items())
+    queued = collected = 0
 
-    def collect(block_index):
-        slot, start = block_index % 2, block_index * B
-        copied[slot].synchronize()
-        for r, d in zip(rows, dst):
-            d[start:start + B] = views[slot, r, :B]
+    def collect(upto):
+        nonlocal collected
+        while collected < upto:
+            slot, start = collected % 2, collected * B
+            copied[slot].synchronize()
+            for r, d in zip(rows, dst):
+                d[start:start + B] = views[slot, r, :B]
+            collected += 1
 
     out, end = dev["out"], 0
-    for block_index in range(data.blocks):
-        if block_index >= 2:
-            collect(block_index - 2)
-        start = block_index * B
-        end = start + B
-        data.draw_sample(slice(start, end))
-        data.evaluate_device(dev["q"], B, pm, out, out.shape[1], stream=stream)
-        ctx.block_sums(out, out.shape[1], B, pm, data.delta_beta if pm else 1.0, sums_all[block_index], stream)
-        slot = block_index % 2
-        if host.shape[2] == out.shape[1]:
-            host[slot].copy_(out, non_blocking=True)
-        else:
-            for r in rows:
-                host[slot, r, :B].copy_(out[r, :B], non_blocking=True)
-        if block_index == data.blocks - 1:
-            sums_host.copy_(sums_all, non_blocking=True)
-        copied[slot].record(stream)
-    for block_index in range(max(0, data.blocks - 2), data.blocks):
-        collect(block_index)
+    result.block_sums = np.zeros((data.blocks, _native.NUM_SUMS))
+    try:
+        for block_index in range(data.blocks):
+            collect(block_index if own else block_index - 1)
+            start = block_index * B
+            end = start + B
+            data.draw_sample(slice(start, end))
+            data.evaluate_device(dev["q"], B, pm, out, out.shape[1], stream=stream)
+            ctx.block_sums(out, out.shape[1], B, pm, data.delta_beta if pm else 1.0, sums_all[block_index], stream)
+            slot = block_index % 2
+            if host.shape[2] == out.shape[1]:
+                host[slot].copy_(out, non_blocking=True)
+            else:
+                for r in rows:
+                    host[slot, r, :B].copy_(out[r, :B], non_blocking=True)
+            if block_index == data.blocks - 1:
+                sums_host.copy_(sums_all, non_blocking=True)
+            copied[slot].record(stream)
+            queued = block_index + 1
+    finally:  # also when a step raises: the blocks before it are the caller's
+        collect(queued)
     result.block_sums = sums_host.numpy().copy()
     if result.path_root is not None:
         result.save_results(end)
