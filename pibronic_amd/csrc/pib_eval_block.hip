@@ -554,7 +554,7 @@ hipError_t launch_s(int pm, const BlockArgs& a, hipStream_t s) {
 
 }  // namespace
 
-hipError_t launch_eval_block(int pm, const BlockArgs& a, hipStream_t s) {
+static hipError_t launch_piece(int pm, const BlockArgs& a, hipStream_t s) {
   switch (a.S) {
 #define PIB_CASE(s_) \
   case s_: return launch_s<s_>(pm, a, s);
@@ -563,6 +563,20 @@ hipError_t launch_eval_block(int pm, const BlockArgs& a, hipStream_t s) {
 #undef PIB_CASE
   }
   return hipErrorInvalidValue;
+}
+
+// A launch has fewer than 2^32 threads: 2^24 waves at a time (2^26 samples of one stream each).
+hipError_t launch_eval_block(int pm, const BlockArgs& a, hipStream_t s) {
+  const int64_t most = (int64_t)(4 / a.C) << 24, NP = (int64_t)a.N * a.P;
+  for (int64_t b = 0; b < a.B; b += most) {
+    BlockArgs p = a;
+    p.B = a.B - b < most ? a.B - b : most;
+    if (a.qf) p.qf += b * NP; else p.q += b * NP;
+    p.out += b;
+    if (a.dbg) p.dbg += b * a.P * eval_debug_record(a.A, a.AR);
+    if (hipError_t e = launch_piece(pm, p, s)) return e;
+  }
+  return hipSuccess;
 }
 
 // The constants in the order the kernel's operands read them (BlockArgs), for the plain or the
