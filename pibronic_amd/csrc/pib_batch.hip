@@ -339,12 +339,25 @@ int pib_batch_create(int n, pib_ctx* const* ctxs, int64_t B, int flags, double d
               : b->lane_ok            ? PIB_BATCH_LANES
               : b->wide_ok            ? PIB_BATCH_WIDE
                                       : PIB_BATCH_SEQUENTIAL;
-  // the persistent lanes kernel's problems share the chip: as many waves as one block of all their
-  // samples needs
-  if (b->family == PIB_BATCH_LANES)
-    for (int i = 0; i < n; ++i) b->lanes[i] = auto_lanes(ctxs[i], B * n, false, true);
-  b->tile_waves = b->family == PIB_BATCH_LANES ? 1 : 4;
-  b->grid_waves = b->num_cu * 8;
+  // The persistent lanes kernel's problems share the chip: as many waves as one block of all their
+  // samples needs. Up to 8 beads per lane and one-wave tiles where the beads are dear (a wave's last ones
+  // hide behind other problems' tiles), up to 4 and, once each of the grid's waves has two, tiles of four
+  // waves where they are cheap against fetching a tile. MI355X, us per block, 8 beads and one-wave tiles /
+  // 4 beads and tiles of four, n temperatures of P = 128..26 and N = 2A: A = 2, n = 2, 16,384 samples
+  // 166 / 146, n = 8, 8,192 236 / 194, with +-dbeta 240 / 234; A = 4, n = 2, 16,384 291 / 224, n = 8, 8,192
+  // 413 / 393, with +-dbeta n = 2, 8,192 204 / 225, n = 8, 8,192 482 / 534; A = 5 with +-dbeta, n = 8,
+  // 8,192 929 / 1,074; A = 6, n = 8, 8,192 745 / 819, 16,384 1,342 / 1,468.
+  b->tile_waves = 4;
+  b->grid_waves = b->num_cu * kBatchWavesPerCU;
+  if (b->family == PIB_BATCH_LANES) {
+    const bool cheap = b->A <= (b->pm ? 2 : 4);
+    int64_t waves = 0;
+    for (int i = 0; i < n; ++i) {
+      b->lanes[i] = auto_lanes(ctxs[i], B * n, false, cheap ? 4 : 8);
+      waves += (B * b->lanes[i] + kWave - 1) / kWave;
+    }
+    if (!cheap || waves < 2 * b->grid_waves) b->tile_waves = 1;
+  }
   PIB_BHIP(b, hipStreamCreateWithFlags(&b->cap, hipStreamNonBlocking));
   return build_schedule(b);
 }

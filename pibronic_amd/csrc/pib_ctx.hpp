@@ -139,7 +139,9 @@ inline bool finite_all(const double* v, size_t n) {
   return true;
 }
 
-inline int auto_lanes(const pib_ctx* c, int64_t B, bool fp32, bool batched = false) {
+constexpr int kBatchWavesPerCU = 8;  // default grid of the persistent batched kernels
+
+inline int auto_lanes(const pib_ctx* c, int64_t B, bool fp32, int batch_beads = 0) {
   // The fewest lanes per sample (a power of two, each doubling adds a level to the cross-lane
   // product tree) that give the launch enough waves and each lane at most kmax beads. The FP64
   // kernel at A >= 7 runs one wave per SIMD (its register budget): 8 waves per SIMD and up to 8
@@ -148,13 +150,14 @@ inline int auto_lanes(const pib_ctx* c, int64_t B, bool fp32, bool batched = fal
   // 1e5 2.25/1.81/1.93/2.29; FP64 A=4, N=8, P=64, 65,536 0.62/0.30/0.19/0.21, 1e5
   // 0.98/0.46/0.29/0.33; FP64 A=6, N=12, P=128, 1e5 2.95/2.69/1.46/1.39; FP32 A=6, N=12, P=128,
   // 1e5 2.86/2.65/1.34/0.83; FP32 A=8, N=16, P=64, 65,536 1.30/0.68/0.57/0.63. Never more lanes
-  // per sample than beads, so that each lane owns at least one bead. In the persistent batched
-  // kernel (B the samples of all its problems) a wave's last beads hide behind other problems'
-  // tiles, so lanes take up to 8 beads there too: sixteen temperatures of A=6, N=12, P=52..256,
-  // 16,384 samples each, 4.12 / 3.90 ms with up to 4 / 8.
+  // per sample than beads, so that each lane owns at least one bead.
+  // batch_beads: the persistent batched kernel (B the samples of all its problems), whose waves take up
+  // to so many beads per lane (pib_batch_create) and which needs no more of them than its grid holds: beyond
+  // that each wave costs the fetch of another tile (two temperatures of A=2, N=4, P=128 and 55, 8,192
+  // samples each: 217 us per block with 64 and 32 lanes, 125 with 16 and 8).
   const bool one_wave = !fp32 && c->A >= 7;
-  const int64_t target = (int64_t)c->num_cu * 4 * kWave * (one_wave ? 8 : 16);
-  const int kmax = one_wave || batched ? 8 : 4;
+  const int64_t target = (int64_t)c->num_cu * kWave * (one_wave ? 32 : batch_beads ? kBatchWavesPerCU : 64);
+  const int kmax = batch_beads ? batch_beads : one_wave ? 8 : 4;
   int maxg = 1;
   while (maxg < 64 && maxg * 2 <= c->P) maxg *= 2;
   int g = 1;
