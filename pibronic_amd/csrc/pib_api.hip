@@ -762,7 +762,7 @@ static int gemm_impl(pib_ctx* c, int bf16x3, int ta, int tb, int64_t M, int64_t 
     g.kchunk = K / splits;
     g.partial = (float*)c->work.p;
   }
-  hipError_t e = launch_gemm_f32(ta != 0, tb != 0, g, (hipStream_t)stream);
+  hipError_t e = launch_gemm_f32(ta != 0, tb != 0, g, c->num_cu, (hipStream_t)stream);
   if (e != hipSuccess) return hip_fail(c, e, "gemm_f32 launch");
   return PIB_OK;
 }
@@ -921,13 +921,13 @@ int pib_flow_whiten(pib_ctx* c, int mode, int64_t B, const void* in, float* work
     if ((e = launch_flow_pre(FLOW_UNWHITEN, ba, in, Y, s)) != hipSuccess) return hip_fail(c, e, "flow pre");
     // X = Y U^T : B operand U transposed (B(k, p) = U[p][k])
     GemmArgs g{Y, U, X, nullptr, nullptr, B * N, P, P, P, P, P, 0, 0, 0};
-    if ((e = launch_gemm_f32(false, true, g, s)) != hipSuccess) return hip_fail(c, e, "flow gemm");
+    if ((e = launch_gemm_f32(false, true, g, c->num_cu, s)) != hipSuccess) return hip_fail(c, e, "flow gemm");
     if ((e = launch_flow_post(FLOW_UNWHITEN, ba, X, out, s)) != hipSuccess) return hip_fail(c, e, "flow post");
   } else {
     const int pre = mode == PIB_FLOW_WHITEN ? FLOW_WHITEN : FLOW_GRAD;
     if ((e = launch_flow_pre(pre, ba, in, X, s)) != hipSuccess) return hip_fail(c, e, "flow pre");
     GemmArgs g{X, U, Y, nullptr, nullptr, B * N, P, P, P, P, P, 0, 0, 0};
-    if ((e = launch_gemm_f32(false, false, g, s)) != hipSuccess) return hip_fail(c, e, "flow gemm");
+    if ((e = launch_gemm_f32(false, false, g, c->num_cu, s)) != hipSuccess) return hip_fail(c, e, "flow gemm");
     if ((e = launch_flow_post(pre, ba, Y, out, s)) != hipSuccess) return hip_fail(c, e, "flow post");
   }
   return PIB_OK;

@@ -22,7 +22,7 @@ struct GemmArgs {
   int bf16x3;  // 1: BF16x3 split on the bf16 matrix cores (K a multiple of 32)
 };
 
-hipError_t launch_gemm_f32(bool ta, bool tb, const GemmArgs& g, hipStream_t s);
+hipError_t launch_gemm_f32(bool ta, bool tb, const GemmArgs& g, int num_cu, hipStream_t s);
 
 // BF16x3 product of pre-split operands (bf16 bits as unsigned short): A hi/lo M x K (lda),
 // B hi/lo stored N x K (ldb); output FP32 C (ldc) and/or split hi/lo (ldo); bias, relu.

@@ -246,7 +246,7 @@ __global__ void __launch_bounds__(256) k_gemm_bf16x3(GemmArgs g) {
 // 16-byte aligned operands: the pipelined tiles of pib_gemm3.hpp. MI355X, us with slabs of 32 in one
 // buffer and 2- and 8-byte LDS writes / these: 2,048 x 1,024 x 256 16.0 / 11.8, 32,768 x 256 x 512 84.7 / 61.2,
 // 2,048 x 256 x 1,024 (B transposed) 19.0 / 15.1, 512 x 256 x 32,768 (A transposed) 172 / 78.
-template <bool TA, bool TB>
+template <bool TA, bool TB, int BUFS>
 __global__ void __launch_bounds__(256) k_gemm_bf16x3_v(GemmArgs g) {
   extern __shared__ __align__(16) unsigned char lds3[];
   const int t = threadIdx.x, lane = t & 63, wr = t >> 7, wc = (t >> 6) & 1;
@@ -256,21 +256,28 @@ __global__ void __launch_bounds__(256) k_gemm_bf16x3_v(GemmArgs g) {
   const float* pa = TA ? g.A + m0 + (t & 63) : g.A + (m0 + (t >> 3)) * g.lda;
   const float* pb = TB ? g.B + (n0 + (t >> 3)) * g.ldb : g.B + n0 + (t & 63);
   f32x4t acc[2][2];
-  tile3<TA, !TB>(pa, g.lda, pb, g.ldb, kbeg, kend, t, (Stage3*)lds3, acc);
-  float* P = g.partial ? g.partial + (int64_t)blockIdx.z * g.M * g.N : nullptr;
+  tile3<TA, !TB, BUFS>(pa, g.lda, pb, g.ldb, kbeg, kend, t, (Stage3*)lds3, acc);
+  if (g.partial) {
+    float* P = g.partial + (int64_t)blockIdx.z * g.M * g.N;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const int64_t col = n0 + wc * 32 + j * 16 + (lane & 15);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) P[(m0 + wr * 32 + i * 16 + 4 * (lane >> 4) + r) * g.N + col] = acc[i][j][r];
+      }
+    return;
+  }
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       const int64_t col = n0 + wc * 32 + j * 16 + (lane & 15);
-      const float bv = !P && g.bias ? g.bias[col] : 0.f;
+      const float bv = g.bias ? g.bias[col] : 0.f;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int64_t row = m0 + wr * 32 + i * 16 + 4 * (lane >> 4) + r;
-        if (P) {
-          P[row * g.N + col] = acc[i][j][r];
-          continue;
-        }
         float v = acc[i][j][r] + bv;
         if (g.relu) v = v > 0.f ? v : 0.f;
         if (g.mask) v = g.mask[row * g.ldmask + col] > 0.f ? v : 0.f;
@@ -280,12 +287,21 @@ __global__ void __launch_bounds__(256) k_gemm_bf16x3_v(GemmArgs g) {
     }
 }
 
-template <bool TA, bool TB>
-static hipError_t launch_x3_v(const GemmArgs& g, dim3 grid, hipStream_t s) {
+template <bool TA, bool TB, int BUFS>
+static hipError_t launch_x3_bufs(const GemmArgs& g, dim3 grid, hipStream_t s) {
   static unsigned long long lds_set = 0;
-  if (hipError_t e = ensure_dynamic_lds((const void*)k_gemm_bf16x3_v<TA, TB>, kTile3Lds, lds_set)) return e;
-  hipLaunchKernelGGL((k_gemm_bf16x3_v<TA, TB>), grid, dim3(256), kTile3Lds, s, g);
+  constexpr size_t lds = BUFS * sizeof(Stage3);
+  if (hipError_t e = ensure_dynamic_lds((const void*)k_gemm_bf16x3_v<TA, TB, BUFS>, lds, lds_set)) return e;
+  hipLaunchKernelGGL((k_gemm_bf16x3_v<TA, TB, BUFS>), grid, dim3(256), lds, s, g);
   return hipGetLastError();
+}
+// Two stages while no more than two work-groups per CU want a place. MI355X, us with one / two: 2,048 x
+// 1,024 x 256 10.0 / 9.7, 256 x 256 x 65,536 84 / 82, 512 x 256 x 256 7.5 / 7.3; 32,768 x 256 x 64 14.5 /
+// 17.7, x 512 49 / 59, 65,536 x 1,024 x 256 185 / 232.
+template <bool TA, bool TB>
+static hipError_t launch_x3_v(const GemmArgs& g, int num_cu, dim3 grid, hipStream_t s) {
+  if ((int64_t)grid.x * grid.y * grid.z > 2 * num_cu) return launch_x3_bufs<TA, TB, 1>(g, grid, s);
+  return launch_x3_bufs<TA, TB, 2>(g, grid, s);
 }
 
 static bool aligned16(const void* p, int64_t ld) {
@@ -297,7 +313,7 @@ bool gemm_shape_ok(const GemmArgs& g) {
   return g.M > 0 && g.N > 0 && g.K > 0 && g.M % kTM == 0 && g.N % kTN == 0 && g.K % kq == 0;
 }
 
-hipError_t launch_gemm_f32(bool ta, bool tb, const GemmArgs& g, hipStream_t s) {
+hipError_t launch_gemm_f32(bool ta, bool tb, const GemmArgs& g, int num_cu, hipStream_t s) {
   if (!gemm_shape_ok(g)) return hipErrorInvalidValue;
   const int splits = g.partial ? (int)(g.K / g.kchunk) : 1;
   const int64_t kq = g.bf16x3 ? kTK3 : kTK;
@@ -305,10 +321,10 @@ hipError_t launch_gemm_f32(bool ta, bool tb, const GemmArgs& g, hipStream_t s) {
   const dim3 grid((unsigned)(g.N / kTN), (unsigned)(g.M / kTM), (unsigned)splits);
   hipError_t ve = hipSuccess;
   if (g.bf16x3 && aligned16(g.A, g.lda) && aligned16(g.B, g.ldb)) {
-    if (!ta && !tb) ve = launch_x3_v<false, false>(g, grid, s);
-    else if (!ta && tb) ve = launch_x3_v<false, true>(g, grid, s);
-    else if (ta && !tb) ve = launch_x3_v<true, false>(g, grid, s);
-    else ve = launch_x3_v<true, true>(g, grid, s);
+    if (!ta && !tb) ve = launch_x3_v<false, false>(g, num_cu, grid, s);
+    else if (!ta && tb) ve = launch_x3_v<false, true>(g, num_cu, grid, s);
+    else if (ta && !tb) ve = launch_x3_v<true, false>(g, num_cu, grid, s);
+    else ve = launch_x3_v<true, true>(g, num_cu, grid, s);
   } else if (g.bf16x3) {
     if (!ta && !tb) hipLaunchKernelGGL((k_gemm_bf16x3<false, false>), grid, dim3(256), 0, s, g);
     else if (!ta && tb) hipLaunchKernelGGL((k_gemm_bf16x3<false, true>), grid, dim3(256), 0, s, g);

@@ -3,8 +3,9 @@
 // accumulator takes lo hi, hi lo, hi hi on v_mfma_f32_16x16x32_bf16 (the dropped lo lo term leaves
 // ~2^-16 relative error per product).
 //
-// K advances in stages of 64, two stages in LDS: the next stage's loads are in flight during the products of
-// the current one, and its conversion meets one barrier per stage. Every thread converts 8
+// K advances in stages of 64: the next stage's loads are in flight during the products of the current one.
+// BUFS = 2 stages in LDS let its conversion meet one barrier per stage; with BUFS = 1 twice as many
+// work-groups fit on a CU (four of 37 KB), the better use where there are as many. Every thread converts 8
 // consecutive k of one row at a time, so both parts go to LDS as 16-byte writes whatever the
 // operand's order in memory (k-contiguous rows by two float4, k-strided columns by 8 coalesced
 // dwords); rows of 72 bf16 (36 banks) keep the 16-byte reads and writes of 16 lanes apart.
@@ -24,7 +25,6 @@ constexpr int kTile3 = 64, kStage3 = 64, kRow3 = kStage3 + 8;
 struct Stage3 {  // one stage of both operands
   unsigned short Ah[kTile3][kRow3], Al[kTile3][kRow3], Bh[kTile3][kRow3], Bl[kTile3][kRow3];
 };
-constexpr size_t kTile3Lds = 2 * sizeof(Stage3);
 
 // A thread's 16 values of a stage: two runs of 8 consecutive k.
 // KS (k strided): p = the thread's column (t % 64) at k = 0; else p = its row (t / 8) at k = 0, its
@@ -107,7 +107,7 @@ __device__ __forceinline__ void products3(const Stage3& s, int t, int slabs, f32
 
 // A tile's sum over [kbeg, kend), a multiple of 32. KSA / KSB: the operand is strided in k; pa / pb:
 // the thread's column or row (see load3).
-template <bool KSA, bool KSB>
+template <bool KSA, bool KSB, int BUFS>
 __device__ __forceinline__ void tile3(const float* __restrict__ pa, int64_t lda, const float* __restrict__ pb,
                                       int64_t ldb, int64_t kbeg, int64_t kend, int t, Stage3* lds,
                                       f32x4t (&acc)[2][2]) {
@@ -125,14 +125,19 @@ __device__ __forceinline__ void tile3(const float* __restrict__ pa, int64_t lda,
   put(lds[0]);
   __syncthreads();
   int b = 0;
-  for (int64_t k0 = kbeg; k0 < kend; k0 += kStage3, b ^= 1) {
+  for (int64_t k0 = kbeg; k0 < kend; k0 += kStage3) {
     const bool more = k0 + kStage3 < kend;
     if (more) {
       load3<KSA>(pa, lda, k0 + kStage3, kend, t, va);
       load3<KSB>(pb, ldb, k0 + kStage3, kend, t, vb);
     }
     products3(lds[b], t, kend - k0 >= kStage3 ? 2 : 1, acc);
-    if (more) put(lds[b ^ 1]);
+    if (!more) break;  // uniform
+    if constexpr (BUFS == 2)
+      b ^= 1;
+    else
+      __syncthreads();  // the stage has been read
+    put(lds[b]);
     __syncthreads();
   }
 }
