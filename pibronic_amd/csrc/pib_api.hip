@@ -110,26 +110,63 @@ int rebuild_block_table(pib_ctx* c) {
   return PIB_OK;
 }
 
-// The block kernel takes every (A, A_rho) without a lanes kernel (without +-dbeta up to eight
-// surfaces), and of those with one the sizes where it is the faster: A = 8, with +-dbeta (three ring
-// chains in one lane's registers) A = 7, and below certain batches, where lanes kernels of one or two
-// waves per SIMD leave the chip waiting, A = 7 (160 samples per CU) and with +-dbeta A = 6 (256) and A = 5
-// (128), unless the caller has set the lanes per sample. Measured (MI355X, us, lanes / block, N = 2 A, P = 64):
-// A = 8 1,000 samples 46 / 27, 16,384 388 / 237, 1e5 1650 / 1416; with +-dbeta 1e5 5470 / 1882; A = 7
-// 700 33 / 23, 8,000 207 / 108, 32,000 501 / 397, 64,000 798 / 780 (N = 3, 47,000 block step 464 / 470), 1e5
-// 1179 / 1290, with +-dbeta 16,384 837 / 286, 1e5
-// 3163 / 1706; A = 6 3,000 39 / 43, 1e5 732 / 1235, with +-dbeta 700 47 / 26, 16,000 563 / 261, 64,000
-// 1286 / 982, 80,000 1115 / 1220; A = 5 3,000 29 / 38, with +-dbeta 700 29 / 24, 32,000 702 / 452, 45,000
-// 573 / 616.
+// Where sizes with a lanes kernel take the block kernel: A = 8 and, with +-dbeta (three ring chains in one
+// lane's registers), A = 7 always; below certain batches, where lanes kernels of one or two waves per
+// SIMD leave the chip waiting, A = 7 and with +-dbeta A = 5 and 6, unless the caller has set the lanes per
+// sample. The lanes kernel spreads a long row over up to 64 lanes and this one over four streams at most,
+// and rows that fill no step of four beads cost it a whole one: the lines below follow both, and the
+// lanes kernel's modes (from about 20 of them at A = 7 its coordinates no longer stay in the L2). Measured
+// (MI355X, time / the lanes kernel's), A, N P samples:
+// 5 with +-dbeta: 8 64 16,000 0.64, 32,768 1.1; 8 100 1,000 1.12, 4,000 0.87; 8 128 4,000 1.03; 8 200 16,000 1.16;
+//   3 6 8,000 0.84, 16,000 1.41; 8 12 16,000 1.04, 24 12 16,000 0.82
+// 6 with +-dbeta: 8 64 40,960 0.70, 65,536 1.04; 8 12 65,536 0.68; 8 200 100 0.82, 1,000 1.10, 16,000 0.80;
+//   8 256 1,000 1.18, 16,000 0.99; 3 3 16,000 0.82, 32,000 1.36
+// 7: 8 64 32,000 0.81, 40,960 1.06, 24 64 40,960 0.47; 8 128 16,000 0.78, 32,000 1.05; 8 128 1,000 1.10, 2,000 0.88;
+//   3 256 16,000 1.09; 3 6 8,000 0.72, 16,000 1.12
+// 8: 1e5 0.86, 16,384 0.61; with +-dbeta 0.34
+static bool block_over_lanes(const pib_ctx* c, bool pm, int64_t B) {
+  const int A = c->A, N = c->N, P = c->P;
+  const int64_t cu = c->num_cu;
+  if (A >= (pm ? 7 : 8)) return true;
+  if (A < (pm ? 5 : 7) || c->lanes) return false;
+  const bool many = A == 7 && N >= 20;
+  int64_t most;  // the lanes kernel's split changes at powers of two: one of them is on either side
+  if (A == 5) most = cu * 128;
+  else if (A == 6) most = cu * 256 + (P < 48 || P > 96);
+  else most = many || P < 48 ? cu * 160 + 1 : cu * (P > 100 ? 64 : 128);
+  const int far = A == 5 ? 64 : A == 6 ? 224 : 112;  // longer rows need enough samples,
+  const int farther = A == 5 ? 112 : A == 6 || N >= 14 ? 256 : 224;  // these stay with the lanes
+  const bool shorts = A == 5 ? P < 9 || (P < 16 && N < 12) : A == 6 ? P < 5 : P < (N < 8 ? 8 : 5);
+  if (B >= most) return false;
+  if (many) return true;
+  if (P > farther || (P > far && B < 8 * cu)) return false;
+  return !shorts || B <= cu * (A == 6 ? 250 : 187) / P;
+}
+
+// And sizes without one, against the one-wave-per-sample kernel: up to eight surfaces, and with +-dbeta
+// all but the following. A wave's exponentials cost the same whatever its samples' modes and at S = 13..16 are
+// the dearer ones (64 products of 4 x 4 blocks and registers that spill), the other kernel's grow with A;
+// the couplings of many modes are where that kernel loses. Measured (time / the one-wave kernel's) with
+// +-dbeta, A A_rho, N P samples: 12 12, 3 3 500 1.27, 2,000 0.89, 30,000 0.45; 16 16, 3 8 1,000 0.99, 3,000 1.16; 3 64
+// 500 0.78, 3,000 1.07, 30,000 0.94; 8 12 500 0.87, 3,000 1.02; 24 8 500 1.09, 2,000 0.75; 24 128 3,000 0.68; 4 16, 10 64
+// 3,000 2.04; 3 12, 3 12 300 0.85, 3,000 1.16, 30,000 0.87;
+// 6 16, 10 64 300 0.90, 3,000 1.35; 6 13, 3 12 3,000 1.59, 10 64 3,000 1.00; 9 16, 10 64 3,000 1.08.
+static bool block_over_wide(const pib_ctx* c, bool pm, int64_t B) {
+  const int A = c->A, N = c->N, P = c->P, S = block_size(A, c->set_A[SET_RHO]);
+  const int64_t cu = c->num_cu;
+  if (!pm) return S <= 8;
+  if (S <= 12) return A <= 4 && S > 8 && P < 20 ? B < 8 * cu || B > 32 * cu : P > 4 || B >= 3 * cu;
+  if (A <= 4 || (A <= 8 && (N < 8 || (S >= 14 && B >= 8 * cu)))) return false;
+  if (P < 12) return B >= cu * (N >= 8 ? 8 : 100);
+  return N >= 8 || B <= 4 * cu || B >= 40 * cu || (S <= 14 && P >= 32);
+}
+
 bool uses_block(const pib_ctx* c, int flags, int64_t B) {
   const bool pm = (flags & PIB_EVAL_PM) != 0;
   if (!c->block_ok[pm] || (flags & (PIB_EVAL_WIDE | PIB_EVAL_FP32 | PIB_EVAL_BF16X3))) return false;
   for (int s = 0; s < (pm ? 4 : 2); ++s)
     if (!c->pref_positive[s]) return false;  // it works with log F_a
-  if (!eval_supported(c->A, c->set_A[SET_RHO])) return pm || block_size(c->A, c->set_A[SET_RHO]) <= 8;
-  if (c->A >= (pm ? 7 : 8)) return true;
-  if (c->lanes) return false;
-  return B <= (int64_t)c->num_cu * (pm ? (c->A == 6 ? 256 : c->A == 5 ? 128 : 0) : (c->A == 7 ? 160 : 0));
+  return eval_supported(c->A, c->set_A[SET_RHO]) ? block_over_lanes(c, pm, B) : block_over_wide(c, pm, B);
 }
 
 // Bead streams per sample (1, 2 or 4) of the block kernel: more of them fill the chip with fewer

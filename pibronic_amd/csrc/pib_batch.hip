@@ -308,7 +308,7 @@ int pib_batch_create(int n, pib_ctx* const* ctxs, int64_t B, int flags, double d
     const int A = c->A, AR = b->args[i].AR;
     b->wide[i] = wide;
     if (wide) b->seq_lanes = false;
-    all_block = all_block && (uses_block(c, flags, INT64_MAX) || (wide && !b->pm && wide4_supported(b->args[i], b->num_cu)));
+    all_block = all_block && (uses_block(c, flags, eval_supported(A, AR) ? INT64_MAX : B) || (wide && !b->pm && wide4_supported(b->args[i], b->num_cu)));
     if (wide || (i > 0 && (A != b->A || AR != b->AR))) b->lane_ok = false;
     if (i == 0) { b->A = A; b->AR = AR; }
     if (A > kWideMaxStates || AR > kWideMaxStates) b->wide_ok = false;

@@ -392,8 +392,10 @@ static hipError_t launch_s4(const EvalArgs& a, hipStream_t s) {
 // 159 / 197, 3,000 218 / 199, 8,300 597 / 469, 12,000 806 / 479; 12 24 128 2,000 509 / 571,
 // 3,000 680 / 573, 16,384 3,600 / 1,725; 9 3 12 2,816 45 / 41, 1e5 1,182 / 742; 11 24 60 50,000
 // 5,211 / 2,937. With 13 surfaces and more a product is 64 instructions here and the 4 of the wide kernel
-// are no more cycles.
+// are no more cycles. Rows of fewer than seven beads leave steps empty and need more waves: 12 3 3 2,816
+// 14.9 / 16.5, 11 3 5 2,816 1.07 of the wide kernel's time, 5,000 1.01, 10,000 0.83.
 bool wide4_supported(const EvalArgs& a, int num_cu) {
+  if (a.P < 7 && a.B < (int64_t)num_cu * 20) return false;
   if (a.dbg || (int64_t)a.N * a.P >= (1 << 25) || a.B < (int64_t)num_cu * 11) return false;
   switch (a.A > a.AR ? a.A : a.AR) {
     case 9: return lds4_bytes<9>(a.N) <= kLds4;
