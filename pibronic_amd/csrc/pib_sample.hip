@@ -33,7 +33,7 @@
 namespace pib {
 
 constexpr int kSampleWaves = 4;   // waves per work-group, each independent
-// Beads staged per lane before a write-out: 8 up to 24 beads per row, else 16 (a whole 128-byte line
+// Beads staged per lane before a write-out: 8 up to 24 beads per row (see also below), else 16 (a whole 128-byte line
 // where rows start on one), or 32 where rows start off a line and the launch writes more than the
 // 256 MB of the memory-side cache. Half lines written apart reach memory one by one once the rows in
 // flight exceed the L2, and so do the two ends of a run off the line, fewer in longer runs; short rows
@@ -53,6 +53,9 @@ static int chunk_for(const SampleArgs* a, int n) {
     if (a[i].P > longest) longest = a[i].P;
   }
   if (longest <= 24) return 8;
+  // in a small launch a last piece of 8 to 15 beads (written out with divisions) costs more than half lines do:
+  // 3 28 2,000 7.9 / 8.5, 12 25 2,000 8.0 / 8.5, 3 28 20,000 9.6 / 10.2 with 8 / 16; 12 28 20,000 19.9 / 18.7
+  if (longest < 48 && longest % 16 >= 8 && all < 16 * 1048576.0) return 8;
   return all > 256 * 1048576.0 && 2.0 * off > all ? 32 : 16;
 }
 
