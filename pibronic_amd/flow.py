@@ -243,7 +243,10 @@ class Flow:
             return [slice(0, B)]
         launch = 128 * self.num_cu
         step = max(1, (128 << 20) // (4 * self.D * launch)) * launch
-        return [slice(b, min(b + step, B)) for b in range(0, B, step)]
+        starts = list(range(0, B, step))
+        if B - starts[-1] <= launch // 2:  # a small rest goes with the piece before it
+            starts.pop()
+        return [slice(b, e) for b, e in zip(starts, starts[1:] + [B])]
 
     def _split_weights_frag(self, stream):
         """bf16 weights (hi parts) in the fragment order of pib_flow_layer_fused_frag, inputs in
@@ -308,10 +311,11 @@ class Flow:
         if fast:
             self._split_weights(stream)
         if fast and self._fused_ok(B, single_bf16):
-            for rows in self._chunks(B) if single_bf16 else [slice(0, B)]:
-                z, ld = zp[rows], logdet[rows]
+            pieces = self._chunks(B) if single_bf16 else [slice(0, B)]
+            for rows in pieces:
+                z, ld = (zp, logdet) if len(pieces) == 1 else (zp[rows], logdet[rows])
                 for l in range(self.layers):
-                    self._layer_fused(False, l, z, z.shape[0], ld, stream, single_bf16)
+                    self._layer_fused(False, l, z, rows.stop - rows.start, ld, stream, single_bf16)
             return
         h1, h2, o = self._buf("h1", (B, h)), self._buf("h2", (B, h)), self._buf("o", (B, D))
         for l in range(self.layers):
@@ -461,18 +465,18 @@ class Flow:
         pieces = [slice(0, B)]
         if layer_events is None and single and self._fused_ok(B, True):
             pieces = self._chunks(B)
-        n = pieces[0].stop
-        zp, work = self._buf("zp", (n, self.D)), self._buf("work", (2 * n * self.D,))
+        most = max(rows.stop - rows.start for rows in pieces)
+        zp, work = self._buf("zp", (most, self.D)), self._buf("work", (2 * most * self.D,))
         for rows in pieces:
             n = rows.stop - rows.start
-            z = zp[:n]
-            self.ctx.flow_draw_base(seed, offset + rows.start, n, z, logrho[rows], stream)
+            z, lr, ld, out = (zp, logrho, logdet, R) if n == B else (zp[:n], logrho[rows], logdet[rows], R[rows])
+            self.ctx.flow_draw_base(seed, offset + rows.start, n, z, lr, stream)
             if layer_events is not None:
                 layer_events[0].record(stream)
-            self._layers_forward(z, n, logdet[rows], stream, single_bf16=single)
+            self._layers_forward(z, n, ld, stream, single_bf16=single)
             if layer_events is not None:
                 layer_events[1].record(stream)
-            self.ctx.flow_whiten(mode, n, z, work, R[rows], stream)
+            self.ctx.flow_whiten(mode, n, z, work, out, stream)
         return R, logrho - logdet
 
 
