@@ -123,8 +123,10 @@ int pib_set_beads(pib_ctx* ctx, int P, double tau);
 int pib_eval_block_flow_offsets(pib_ctx* ctx, const float* dq_dev, int64_t B, int flags, double* out_dev,
                                 int64_t out_stride, void* stream);
 
-/* Lanes cooperating on one sample (power of two <= 64), 0 = automatic. Tuning only. The getter
- * reports the count the FP64 lanes kernel uses for a block of B samples. */
+/* Lanes cooperating on one sample (power of two <= 64), 0 = automatic. Tuning only: lanes that are
+ * set keep sizes which small batches take to the block kernel (A = 7, with +-dbeta A = 5 and 6)
+ * in the lanes kernel; A = 8, with +-dbeta A = 7, and A > 8 have no lanes kernel and ignore them. The
+ * getter reports the count the FP64 lanes kernel uses for a block of B samples. */
 int pib_set_lanes_per_sample(pib_ctx* ctx, int lanes);
 int pib_get_lanes_per_sample(pib_ctx* ctx, int64_t B);
 
@@ -136,8 +138,10 @@ int pib_get_lanes_per_sample(pib_ctx* ctx, int64_t B);
  * diagonalize_coupling_matrix and build_numerator (:1062-1213) fused into one launch.
  * debug_dev, if not NULL, receives per (sample, bead) records of
  * [O_rho (A_rho), O_vib (A), S_p, M (A*A)] (unscaled O), B*P records.
- * A <= 8 runs a lanes-per-sample kernel; 8 < A <= 16 (and any A with PIB_EVAL_WIDE) runs one
- * wave per sample with 16x16 padded matrices. A or A_rho > 16: PIB_ERR_UNSUPPORTED. */
+ * By size this runs lanes per sample (A <= 7), four bead streams per wave on 4x4 matrix blocks
+ * (A = 8, +-dbeta from A = 7 on, small batches from A = 5 on), four samples per wave (A = 9..12) or one
+ * wave per sample with 16x16 padded matrices (the rest, and any A with PIB_EVAL_WIDE).
+ * A or A_rho > 16: PIB_ERR_UNSUPPORTED. */
 int pib_eval_block(pib_ctx* ctx, const double* q_dev, int64_t B, int flags, double* out_dev,
                    int64_t out_stride, double* debug_dev, void* stream);
 
@@ -390,8 +394,8 @@ int pib_batch_bind(pib_batch* batch, int i, const double* q_dev, double* out_dev
  * sums_dev + (k * n + i) * PIB_NUM_SUMS (max_blocks * n * PIB_NUM_SUMS doubles). */
 int pib_batch_bind_sums(pib_batch* batch, double* sums_dev);
 
-/* Schedule: kernel family, lanes per sample of every problem (lanes family; NULL keeps the
- * current ones), tile size (waves of the lanes family, samples of the wide family) and the
+/* Schedule: kernel family, lanes per sample of every problem (lanes family, and one launch per
+ * problem as pib_set_lanes_per_sample; NULL keeps the current ones), tile size (waves of the lanes family, samples of the wide family) and the
  * number of persistent waves. */
 int pib_batch_set_schedule(pib_batch* batch, int family, const int* lanes, int tile_waves,
                            int grid_waves);

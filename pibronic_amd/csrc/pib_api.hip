@@ -124,11 +124,11 @@ int rebuild_block_table(pib_ctx* c) {
 // 7: 8 64 32,000 0.81, 40,960 1.06, 24 64 40,960 0.47; 8 128 16,000 0.78, 32,000 1.05; 8 128 1,000 1.10, 2,000 0.88;
 //   3 256 16,000 1.09; 3 6 8,000 0.72, 16,000 1.12
 // 8: 1e5 0.86, 16,384 0.61; with +-dbeta 0.34
-static bool block_over_lanes(const pib_ctx* c, bool pm, int64_t B) {
+static bool block_over_lanes(const pib_ctx* c, bool pm, int64_t B, bool lanes_set) {
   const int A = c->A, N = c->N, P = c->P;
   const int64_t cu = c->num_cu;
   if (A >= (pm ? 7 : 8)) return true;
-  if (A < (pm ? 5 : 7) || c->lanes) return false;
+  if (A < (pm ? 5 : 7) || c->lanes || lanes_set) return false;
   const bool many = A == 7 && N >= 20;
   int64_t most;  // the lanes kernel's split changes at powers of two: one of them is on either side
   if (A == 5) most = cu * 128;
@@ -161,12 +161,12 @@ static bool block_over_wide(const pib_ctx* c, bool pm, int64_t B) {
   return N >= 8 || B <= 4 * cu || B >= 40 * cu || (S <= 14 && P >= 32);
 }
 
-bool uses_block(const pib_ctx* c, int flags, int64_t B) {
+bool uses_block(const pib_ctx* c, int flags, int64_t B, bool lanes_set) {
   const bool pm = (flags & PIB_EVAL_PM) != 0;
   if (!c->block_ok[pm] || (flags & (PIB_EVAL_WIDE | PIB_EVAL_FP32 | PIB_EVAL_BF16X3))) return false;
   for (int s = 0; s < (pm ? 4 : 2); ++s)
     if (!c->pref_positive[s]) return false;  // it works with log F_a
-  return eval_supported(c->A, c->set_A[SET_RHO]) ? block_over_lanes(c, pm, B) : block_over_wide(c, pm, B);
+  return eval_supported(c->A, c->set_A[SET_RHO]) ? block_over_lanes(c, pm, B, lanes_set) : block_over_wide(c, pm, B);
 }
 
 // Bead streams per sample (1, 2 or 4) of the block kernel: more of them fill the chip with fewer
@@ -228,10 +228,10 @@ static BlockArgs block_args(const pib_ctx* c, const EvalArgs& a, bool pm) {
   return b;
 }
 
-hipError_t launch_eval(const pib_ctx* c, int flags, bool wide, const EvalArgs& a, hipStream_t s) {
+hipError_t launch_eval(const pib_ctx* c, int flags, bool wide, const EvalArgs& a, hipStream_t s, bool lanes_set) {
   const int pm = (flags & PIB_EVAL_PM) ? 1 : 0;
   if (flags & PIB_EVAL_FP32) return launch_eval_fp32(a.A, a.AR, pm, a, s);
-  if (uses_block(c, flags, a.B)) return launch_eval_block(pm, block_args(c, a, pm != 0), s);
+  if (uses_block(c, flags, a.B, lanes_set)) return launch_eval_block(pm, block_args(c, a, pm != 0), s);
   if (wide && !pm && !(flags & (PIB_EVAL_WIDE | PIB_EVAL_BF16X3)) && wide4_supported(a, c->num_cu))
     return launch_eval_wide4(a, s);
   if (wide) return launch_eval_wide(pm, a, s, (flags & PIB_EVAL_BF16X3) != 0);

@@ -55,6 +55,7 @@ struct pib_batch {
   // schedule
   int family = 0;  // PIB_BATCH_LANES or PIB_BATCH_WIDE
   std::vector<int> lanes;
+  bool lanes_set = false;  // the caller's (batch_set_schedule) or the tuner's
   int tile_waves = 4, grid_waves = 0;
   int ntiles = 0;
   // caller-owned buffers (pib_batch_bind*), library-owned scratch
@@ -161,7 +162,7 @@ hipError_t launch_batch_eval(pib_batch* b, hipStream_t s) {
   if (b->family == PIB_BATCH_SEQUENTIAL) {  // one launch per problem, tuned lanes
     for (int i = 0; i < b->n; ++i) {
       const EvalArgs& a = b->args[i];
-      const hipError_t e = launch_eval(b->ctx[i], b->flags, b->wide[i], a, s);
+      const hipError_t e = launch_eval(b->ctx[i], b->flags, b->wide[i], a, s, b->lanes_set);
       if (e != hipSuccess) return e;
     }
     return hipSuccess;
@@ -415,6 +416,7 @@ int pib_batch_set_schedule(pib_batch* b, int family, const int* lanes, int tile_
       if (g < 1 || g > 64 || (g & (g - 1))) return bfail(b, PIB_ERR_ARG, "batch_set_schedule: lanes must be powers of two <= 64");
     }
     b->lanes.assign(lanes, lanes + b->n);
+    b->lanes_set = true;
   }
   b->family = family;
   b->tile_waves = tile_waves;
@@ -492,6 +494,7 @@ int pib_batch_tune(pib_batch* b, uint64_t seed, double* best_ms, double* sequent
     int family, kt, tile, grid;
     std::vector<int> lanes;
     double ms;
+    bool lanes_set = true;
   };
   auto lanes_for = [&](int kt) {
     std::vector<int> g(b->n);
@@ -503,7 +506,10 @@ int pib_batch_tune(pib_batch* b, uint64_t seed, double* best_ms, double* sequent
   };
   auto run = [&](Cand& c) -> int {
     b->family = c.family;
-    if (c.family != PIB_BATCH_WIDE) b->lanes = c.lanes;
+    if (c.family != PIB_BATCH_WIDE) {
+      b->lanes = c.lanes;
+      b->lanes_set = c.lanes_set;
+    }
     b->tile_waves = c.tile;
     b->grid_waves = c.grid;
     int r = build_schedule(b);
@@ -517,19 +523,24 @@ int pib_batch_tune(pib_batch* b, uint64_t seed, double* best_ms, double* sequent
     if (fam == PIB_BATCH_LANES && (!b->lane_ok || (b->flags & PIB_EVAL_FP32))) continue;
     if (fam == PIB_BATCH_WIDE && !b->wide_ok) continue;
     Cand cur{fam, 4, 4, b->num_cu * 8, lanes_for(4), 1e300};
+    if (fam == PIB_BATCH_SEQUENTIAL) {  // first with no lanes set: each size in the kernel pib_eval_block takes
+      for (int i = 0; i < b->n; ++i)
+        cur.lanes[i] = auto_lanes(b->ctx[i], b->B, (b->flags & PIB_EVAL_FP32) != 0);
+      cur.lanes_set = false;
+    }
     if (best.family >= 0) {  // prune a family whose default schedule is far behind
       Cand probe = cur;
       if ((rc = run(probe))) return rc;
       if (probe.ms > 1.5 * best.ms) continue;
     }
     if (fam == PIB_BATCH_SEQUENTIAL) {  // per-problem launches: only the lanes matter
-      if (!b->seq_lanes) {
-        if ((rc = run(cur))) return rc;
-      } else {
+      if ((rc = run(cur))) return rc;
+      if (b->seq_lanes) {
         for (int kt : {2, 4, 8, 16}) {
           Cand c = cur;
           c.kt = kt;
           c.lanes = lanes_for(kt);
+          c.lanes_set = true;
           if ((rc = run(c))) return rc;
           if (c.ms < cur.ms) cur = c;
         }
@@ -573,7 +584,10 @@ int pib_batch_tune(pib_batch* b, uint64_t seed, double* best_ms, double* sequent
     if (cur.ms < best.ms) best = cur;
   }
   b->family = best.family;
-  if (best.family != PIB_BATCH_WIDE) b->lanes = best.lanes;
+  if (best.family != PIB_BATCH_WIDE) {
+    b->lanes = best.lanes;
+    b->lanes_set = best.lanes_set;
+  }
   b->tile_waves = best.tile;
   b->grid_waves = best.grid;
   if ((rc = build_schedule(b))) return rc;

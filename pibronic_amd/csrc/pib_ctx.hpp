@@ -174,8 +174,9 @@ namespace pib {
 int make_eval_args(pib_ctx* c, int flags, int64_t B, EvalArgs* a, bool* wide);
 // Launch the evaluation that make_eval_args prepared (flags as given there) with the kernel
 // this context's sizes call for; `a` complete with q (or qf), out, out_stride and dbg.
-hipError_t launch_eval(const pib_ctx* c, int flags, bool wide, const EvalArgs& a, hipStream_t s);
+// lanes_set: the caller has chosen a.G, so sizes with a lanes kernel run in it.
+hipError_t launch_eval(const pib_ctx* c, int flags, bool wide, const EvalArgs& a, hipStream_t s, bool lanes_set = false);
 // Whether launch_eval takes the block kernel for these flags and this many samples (B = INT64_MAX: for
 // any number).
-bool uses_block(const pib_ctx* c, int flags, int64_t B);
+bool uses_block(const pib_ctx* c, int flags, int64_t B, bool lanes_set = false);
 }  // namespace pib
