@@ -1,4 +1,4 @@
-"""Samples share a wave of the block kernel, and each keeps its own scaling of the exponential: a sample
+"""Samples share a wave of the block kernel (and of the four-sample kernel, 10 surfaces), and each keeps its own scaling of the exponential: a sample
 far out (finite coordinates, a large |tau V|) changes no bit of another's outputs. Against the
 one-wave-per-sample kernel on the same coordinates 1e-11, as between any two FP64 kernels."""
 import numpy as np
@@ -10,7 +10,7 @@ from pibronic_amd import pimc
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("A,pm", [(7, True), (8, False), (8, True), (11, True), (15, True)])
+@pytest.mark.parametrize("A,pm", [(7, True), (8, False), (8, True), (11, True), (15, True), (10, False)])
 @pytest.mark.parametrize("far", [1e2, 1e3, 1e5, 1e7, 1e12])
 def test_an_outlier_stays_alone(tmp_path, A, pm, far):
     print(f"[gpu-case] block outlier A={A} pm={pm} far={far:g}", flush=True)
