@@ -141,10 +141,10 @@ __device__ __forceinline__ void sym_mul(const double (&X)[NB][NB], const double 
 // T = exp(X) of the wave's four symmetric matrices, zero outside the leading n x n block (X is
 // scaled in place): Exp16's degree-16 polynomial in four products, scaled and squared. Each stream has
 // its own scaling 2^-s and is squared s times (powers of two are exact), so that its bits are the same
-// whichever samples share the wave; the wave runs the largest count. One count for all four costs less
-// (A = 11, N = 17, P = 50, 3,001 samples with +-dbeta 128 / 133 us, A = 8 the same) and loses up to all
-// digits of a sample beside one whose |tau V| is large. Scaling the coefficients on the scalar unit
-// where the counts agree is slower (A = 8, N = 16, P = 64, 1e5 samples with +-dbeta 1,793 / 1,816 us).
+// whichever samples share the wave; the wave runs the largest count. One count for all four loses up to
+// all digits of a sample beside one whose |tau V| is large and costs little less (MI355X, us, shared / own:
+// A = 8, N = 16, P = 64, 1e5 samples 1,330 / 1,327, with +-dbeta 1,787 / 1,791; A = 11, N = 17, P = 50, 3,001
+// samples with +-dbeta 128.7 / 132.1). Scaling by v_ldexp_f64: products with a per-lane power of two take 1,373 at A = 8.
 // alpha = |X^2|_F^(1/2) needs only its binary exponent: its sum is taken in FP32, of alpha^4 2^-100
 // (alpha up to 2^57 without overflow; below 2^-6, where s is 0 anyway, it may vanish).
 template <int NB>
@@ -179,13 +179,12 @@ __device__ __forceinline__ void expm_block(double (&X)[NB][NB], int n, int i, in
   smax = max(smax, __builtin_amdgcn_update_dpp(smax, smax, 0x128, 0xF, 0xF, false));
   smax = __builtin_amdgcn_readfirstlane(smax);
   if (smax) {
-    const double k1 = __builtin_bit_cast(double, (unsigned long long)(1023 - s) << 52), k2 = k1 * k1;
 #pragma unroll
     for (int I = 0; I < NB; ++I)
 #pragma unroll
       for (int K = 0; K < NB; ++K) {
-        X[I][K] *= k1;
-        X2[I][K] *= k2;
+        X[I][K] = ldexp(X[I][K], -s);
+        X2[I][K] = ldexp(X2[I][K], -2 * s);
       }
   }
 #pragma unroll
@@ -222,12 +221,17 @@ __device__ __forceinline__ void expm_block(double (&X)[NB][NB], int n, int i, in
   sym_mul_upper<NB>(F, G, T);
   mirror<NB>(T, ident);
   for (int k = 0; k < smax; ++k) {
-    sym_mul<NB>(T, T, ident, F);
+#pragma unroll
+    for (int I = 0; I < NB; ++I)
+#pragma unroll
+      for (int K = I; K < NB; ++K) F[I][K] = 0.0;
+    sym_mul_upper<NB>(T, T, F);
     const bool mine = k < s;
 #pragma unroll
     for (int I = 0; I < NB; ++I)
 #pragma unroll
-      for (int K = 0; K < NB; ++K) T[I][K] = mine ? F[I][K] : T[I][K];
+      for (int K = I; K < NB; ++K) T[I][K] = mine ? F[I][K] : T[I][K];
+    mirror<NB>(T, ident);
   }
 }
 
