@@ -141,10 +141,13 @@ __device__ __forceinline__ void sym_mul(const double (&X)[NB][NB], const double 
 // T = exp(X) of the wave's four symmetric matrices, zero outside the leading n x n block (X is
 // scaled in place): Exp16's degree-16 polynomial in four products, scaled and squared. Each stream has
 // its own scaling 2^-s and is squared s times (powers of two are exact), so that its bits are the same
-// whichever samples share the wave; the wave runs the largest count. One count for all four loses up to
-// all digits of a sample beside one whose |tau V| is large and costs little less (MI355X, us, shared / own:
-// A = 8, N = 16, P = 64, 1e5 samples 1,330 / 1,327, with +-dbeta 1,787 / 1,791; A = 11, N = 17, P = 50, 3,001
-// samples with +-dbeta 128.7 / 132.1). Scaling by v_ldexp_f64: products with a per-lane power of two take 1,373 at A = 8.
+// whichever samples share the wave: all are squared up to the wave's smallest count, then those that
+// need more. One count for all four loses up to all digits of a sample beside one whose |tau V| is large.
+// MI355X, us, one count / own: A = 8, N = 16, P = 64, 1e5 samples 1,327 / 1,340, with +-dbeta 1,797 / 1,800,
+// 262,144 of a trained flow (two or three squarings) 3,930 / 4,062; A = 11, N = 17, P = 50, 3,001 samples
+// with +-dbeta 128 / 130; A = 16, N = 10, P = 30, 20,000 with +-dbeta 1,091 / 1,110. (Products with a per-lane
+// power of two instead of v_ldexp_f64: A = 8 1,373; one loop that selects after every squaring: trained
+// flow 4,175.)
 // alpha = |X^2|_F^(1/2) needs only its binary exponent: its sum is taken in FP32, of alpha^4 2^-100
 // (alpha up to 2^57 without overflow; below 2^-6, where s is 0 anyway, it may vanish).
 template <int NB>
@@ -175,9 +178,17 @@ __device__ __forceinline__ void expm_block(double (&X)[NB][NB], int n, int i, in
   const float sd = fmaf(0.25f, __log2f(m), 25.0f - (float)E::log2_theta);
   int s = 0;
   if (sd > 0.0f) s = sd < 64.0f ? (int)ceilf(sd) : 64;
-  int smax = max(s, __builtin_amdgcn_update_dpp(s, s, 0x124, 0xF, 0xF, false));  // the streams: row_ror 4, 8
-  smax = max(smax, __builtin_amdgcn_update_dpp(smax, smax, 0x128, 0xF, 0xF, false));
-  smax = __builtin_amdgcn_readfirstlane(smax);
+  // largest and smallest of the four streams' counts: s and 64 - s in one register, row_ror 4, 8
+  typedef unsigned short us2 __attribute__((ext_vector_type(2)));
+  auto pmax = [](unsigned x, unsigned y) {
+    const us2 p = __builtin_bit_cast(us2, x), q = __builtin_bit_cast(us2, y);
+    return __builtin_bit_cast(unsigned, __builtin_elementwise_max(p, q));
+  };
+  unsigned pk = (unsigned)s | (unsigned)(64 - s) << 16;
+  pk = pmax(pk, (unsigned)__builtin_amdgcn_update_dpp((int)pk, (int)pk, 0x124, 0xF, 0xF, false));
+  pk = pmax(pk, (unsigned)__builtin_amdgcn_update_dpp((int)pk, (int)pk, 0x128, 0xF, 0xF, false));
+  pk = (unsigned)__builtin_amdgcn_readfirstlane((int)pk);
+  const int smax = (int)(pk & 0xffffu), smin = 64 - (int)(pk >> 16);
   if (smax) {
 #pragma unroll
     for (int I = 0; I < NB; ++I)
@@ -220,7 +231,14 @@ __device__ __forceinline__ void expm_block(double (&X)[NB][NB], int n, int i, in
     }
   sym_mul_upper<NB>(F, G, T);
   mirror<NB>(T, ident);
-  for (int k = 0; k < smax; ++k) {
+  for (int k = 0; k < smin; ++k) {
+    sym_mul<NB>(T, T, ident, F);
+#pragma unroll
+    for (int I = 0; I < NB; ++I)
+#pragma unroll
+      for (int K = 0; K < NB; ++K) T[I][K] = F[I][K];
+  }
+  for (int k = smin; k < smax; ++k) {
 #pragma unroll
     for (int I = 0; I < NB; ++I)
 #pragma unroll
