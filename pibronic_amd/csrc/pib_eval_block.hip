@@ -24,16 +24,20 @@
 // Padding: rows and columns >= A of X are zero and the Taylor identity covers only the leading
 // A x A block, so M is zero outside it; padded surfaces have log F = -inf, O = 0.
 //
-// Measured (MI355X, evaluation of 1e5 samples at A = 8, N = 16, P = 64, us): 1327 against 1650 for the
+// Measured (MI355X, evaluation of 1e5 samples at A = 8, N = 16, P = 64, us): 1340 against 1650 for the
 // per-lane kernel (one wave per SIMD, a third of its vector instructions moves to and from the
-// accumulation registers); with +-dbeta 1793 against 5470 for three single-chain passes of that
-// kernel. With +-dbeta at A = 12, N = 24, P = 128, 16,384 samples 1478 against 5720 for the
-// one-wave-per-sample kernel; at A = 11, N = 17, P = 50, 3,001 samples 122 against 373.
+// accumulation registers); with +-dbeta 1800 against 5470 for three single-chain passes of that
+// kernel. With +-dbeta at A = 12, N = 24, P = 128, 16,384 samples 1480 against 5720 for the
+// one-wave-per-sample kernel; at A = 11, N = 17, P = 50, 3,001 samples 130 against 373.
 //
 // What bounds it: FP64 issue. On gfx950 the FP64 matrix and vector instructions share one pipe
 // (timed together they add up exactly: 8 mfma_f64_4x4x4 + 32 v_fma_f64 take 311 cycles per SIMD,
 // alone 152 and 174), so the kernel counts instructions of both kinds; per flop the matrix
-// instructions are the cheaper ones (18.8 cycles per 4x4x4x4, 70 per 16x16x4, 5.4 per v_fma_f64).
+// instructions are the cheaper ones (18.8 cycles per 4x4x4x4, 70 per 16x16x4, 5.4 per v_fma_f64). Memory
+// does not: each step of four beads takes 16 (float offsets) or 32 bytes of a line, so lines come again
+// (8.4 GB for 1.07 GB at 262,144 float offsets, 2.1 TB/s with the writes), and the registers below spill 72 to 84 bytes per
+// lane at S = 8 (0.28 GB written in that launch, once per wave and four steps, outside the exponential),
+// up to 36 at S <= 7, none to 20 at S = 9..12 and 380 to 444 at S = 13..16.
 #include "pib_common.hpp"
 #include "pib_ctx.hpp"
 #include "pib_expm.hpp"
@@ -277,7 +281,7 @@ __device__ __forceinline__ void join(double (&R)[NB][NB], double ident) {
     for (int K = 0; K < NB; ++K) R[I][K] = Z[I][K];
 }
 
-// Registers: at S <= 8 four waves per SIMD (three with +-dbeta), above two.
+// Registers: at S <= 8 four waves per SIMD (three with +-dbeta), above two; what they spill stands above.
 template <int S, bool PM>
 struct BlockOccupancy {
   static constexpr int waves = S <= 8 ? (PM ? 3 : 4) : 2;
