@@ -46,8 +46,9 @@ extern "C" {
 #define PIB_EVAL_PM 1      /* also g(beta +- dbeta): block_compute_pm                     */
 #define PIB_EVAL_NOSCALE 2 /* skip the S12 scaling (S_p = 1), as the explicit golden test */
 #define PIB_EVAL_WIDE 4    /* force the one-wave-per-sample kernel (any A, A_rho <= 16; without
-                              it small blocks of A > 8 without +-dbeta, and prefactors that
-                              are not positive, take it); a tuning/testing switch           */
+                              it the sizes above eight surfaces where it is the faster, and
+                              prefactors that are not positive, take it); a tuning/testing
+                              switch                                                        */
 #define PIB_EVAL_FP32 8    /* reduced precision (A <= 8): O-factors, V, M = exp(-tau V) (a
                               scaled and squared Taylor polynomial) and the ring products in
                               FP32 (power-of-two renormalised); FP64 log-scale and rho
@@ -395,8 +396,8 @@ int pib_batch_bind(pib_batch* batch, int i, const double* q_dev, double* out_dev
 int pib_batch_bind_sums(pib_batch* batch, double* sums_dev);
 
 /* Schedule: kernel family, lanes per sample of every problem (lanes family, and one launch per
- * problem as pib_set_lanes_per_sample; NULL keeps the current ones), tile size (waves of the lanes family, samples of the wide family) and the
- * number of persistent waves. */
+ * problem as pib_set_lanes_per_sample; NULL keeps the current ones), tile size (waves of the lanes
+ * family, samples of the wide family) and the number of persistent waves. */
 int pib_batch_set_schedule(pib_batch* batch, int family, const int* lanes, int tile_waves,
                            int grid_waves);
 int pib_batch_get_schedule(pib_batch* batch, int* family, int* lanes, int* tile_waves,
